@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <string>
 #include <memory>
+#include <utility>
 #include <vector>
 
 #include "../../../include/rm.h"
@@ -54,6 +55,10 @@ struct DevBuf {
         if (n == 0) n = 16;
         RM_HIP(hipMalloc(&ptr, n));
         bytes = n;
+    }
+    void swap(DevBuf& o) {
+        std::swap(ptr, o.ptr);
+        std::swap(bytes, o.bytes);
     }
     template <typename T>
     T* as() const { return static_cast<T*>(ptr); }

@@ -1,5 +1,6 @@
 // Internal entry points behind the C ABI (capi.cpp).
 #pragma once
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -29,8 +30,12 @@ struct TwoLevelBuild {
     uint64_t stored = 0, total = 0;  // triangles stored once per shape, and over all instances
     double seconds = 0;
 };
+// Builds one shape's tree (vertex offset, face offset, face count); false
+// leaves it to the host builder.
+using ShapeBuilder = std::function<bool(uint32_t, uint32_t, uint32_t, Bvh8Build&)>;
 TwoLevelBuild build_two_level(const std::vector<float>& vertices, const std::vector<uint32_t>& indices,
-                              const std::vector<rm_instance_desc>& insts, int threads);
+                              const std::vector<rm_instance_desc>& insts, int threads,
+                              const ShapeBuilder& shape_tree = ShapeBuilder());
 void scene_compile_materials(rm_scene* s, const char* src, size_t len, const char* options, std::string& log);
 void scene_build_envmap(rm_scene* s);
 // Loads the scene's material library with the radiance-cache shading kernel.

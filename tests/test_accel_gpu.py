@@ -1,0 +1,138 @@
+"""Acceleration structures built on the device: the tree has the host
+builder's node count and depth (both choose the same splits), and closest and
+any hits through it equal the oracle's exhaustive search bit for bit, at the
+sizes where the builder's phases meet (64 and 1024 triangles per range, 4096
+per workgroup, the smallest device build) and for geometry that leaves nothing to split on.
+Hits do not depend on the tree, so equality needs no tolerance."""
+import numpy as np
+import pytest
+
+import raymond_amd.api as api
+import raymond_amd.scenes as scenes
+from oracle import binding
+from tests.parity import ORACLE_THREADS, assert_hits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def soup(rng, n):
+    return rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(0, 0.03, (n, 3, 3))
+
+
+def coincident(rng, n):
+    """Triangles whose bounds share one centre: no axis to split on."""
+    t = rng.normal(0, 0.3, (n, 3, 3)).astype(np.float32)
+    t[:, 2] = -t[:, 0]
+    t[:, 1] = 0.0
+    return t
+
+
+def clusters(rng, n):
+    """Cluster distances spanning 12 decades: very uneven splits."""
+    s = 10.0 ** rng.uniform(-8, 4, (n, 1, 1))
+    return s * (rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(0, 0.1, (n, 3, 3)))
+
+
+def flat(rng, n):
+    t = soup(rng, n)
+    t[:, :, 2] = 0.25
+    return t
+
+
+def repeated(rng, n):
+    return np.repeat(soup(rng, 7), (n + 6) // 7, axis=0)[:n]
+
+
+def slivers(rng, n):
+    """A third of the triangles without area."""
+    t = soup(rng, n)
+    t[::3, 2] = t[::3, 1]
+    return t
+
+
+def description(tris, instances=1, seed=0):
+    rng = np.random.default_rng(seed)
+    d = scenes.SceneDescription("soup")
+    d.surface_materials = [scenes.diffuse_material("white", (0.7, 0.7, 0.7))]
+    d.light_materials = [scenes.background_world("world", (0.1, 0.1, 0.1))]
+    d.envmap_resolution = 64
+    v = tris.reshape(-1, 3).astype(np.float32)
+    k = tris.shape[0]
+    ids = []
+    for part in np.array_split(np.arange(k), instances):
+        if part.size:
+            ids.append(d.add_shape(scenes.Shape(v.reshape(-1, 3, 3)[part].reshape(-1, 3),
+                                                np.tile([0.0, 0.0, 1.0], (3 * part.size, 1)),
+                                                np.arange(3 * part.size).reshape(-1, 3), 0)))
+    for j, s in enumerate(ids):
+        m = np.eye(4) if j == 0 else scenes.translate(rng.uniform(-1, 1, 3)) @ scenes.rotate_z(rng.uniform(0, 360))
+        d.add_entity(s, m)
+    d.camera = dict(transform=scenes.look_at((0.0, -4.0, 2.0), (0.0, 0.0, 0.0)), near=1e-3, far=1e4, focal=2.0)
+    return d
+
+
+def world(d):
+    out = []
+    for s, m, _, _ in d.entities:
+        c = np.asarray(m, np.float32)
+        p = d.shapes[s].vertices[d.shapes[s].faces.reshape(-1)]
+        w = [((c[a, 0] * p[:, 0] + c[a, 1] * p[:, 1]) + c[a, 2] * p[:, 2]) + c[a, 3] for a in range(3)]
+        out.append(np.stack(w, 1).astype(np.float32))
+    return np.concatenate(out).reshape(-1, 9)
+
+
+def rays_at(tris, rng, n):
+    t = tris.reshape(-1, 3, 3)
+    target = t[rng.integers(0, t.shape[0], n)].mean(1) + rng.normal(0, 0.02, (n, 3))
+    o = rng.uniform(-2, 2, (n, 3))
+    d = target - o
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    return np.concatenate([o, np.full((n, 1), 1e-3), d, np.full((n, 1), 1e4)], 1).astype(np.float32)
+
+
+CASES = [(soup, 511, 1), (soup, 512, 1), (soup, 1024, 1), (soup, 1025, 3), (soup, 4096, 1), (soup, 4097, 2), (soup, 8193, 1), (soup, 50021, 5),
+         (coincident, 1031, 1), (coincident, 4500, 1), (clusters, 20011, 1), (flat, 4160, 2), (repeated, 4300, 1),
+         (slivers, 3001, 1)]
+
+
+@pytest.mark.parametrize("make,n,instances", CASES, ids=lambda x: getattr(x, "__name__", str(x)))
+def test_device_tree_equals_host_tree(device, make, n, instances):
+    rng = np.random.default_rng(n)
+    d = description(make(rng, n), instances, seed=n)
+    w = world(d)
+    scene = api.Scene(device, d)
+    scene.build_accel()
+    st = scene.stats()
+    assert st.triangles == n
+    if make is not coincident:  # there, halves depend on the order of equal centres
+        assert (st.bvh_nodes, st.bvh_depth) == api.bvh8_check(w)
+    orc = binding.OracleScene(d)
+    rays = rays_at(w, rng, 2000)
+    got = scene.trace_closest(rays)
+    assert_hits_equal(got, orc.trace_closest(rays, brute_force=True, threads=ORACLE_THREADS), rays)
+    short = rays.copy()
+    short[:, 7] = 1.5
+    assert np.array_equal(scene.trace_any(short), orc.trace_any(short, brute_force=True, threads=ORACLE_THREADS))
+
+
+@pytest.mark.parametrize("n", [512, 5000])
+def test_two_level_shapes_built_on_the_device(device, n):
+    rng = np.random.default_rng(n)
+    d = description(soup(rng, n), 1)
+    d.add_entity(0, scenes.translate((0.4, 0.1, 0.2)) @ scenes.scale((0.5, 0.5, 0.5)))
+    scene = api.Scene(device, d)
+    scene.build_accel(two_level=True)
+    assert (scene.stats().stored_triangles, scene.stats().triangles) == (n, 2 * n)
+    orc = binding.OracleScene(d)
+    orc.set_two_level(True)
+    rays = rays_at(world(d), rng, 2000)
+    assert_hits_equal(scene.trace_closest(rays), orc.trace_closest(rays, threads=ORACLE_THREADS), rays)
+
+
+def test_geometry_that_is_not_finite_takes_the_host_builder(device):
+    """The device builder hands it over; the host builder's answer stands."""
+    tris = soup(np.random.default_rng(5), 1500)
+    tris[700, 1, 2] = np.inf
+    d = description(tris, 1)
+    with pytest.raises(api.RmError, match="quantisation failed"):
+        api.Scene(device, d).build_accel()
