@@ -60,6 +60,10 @@ struct DevBuf {
         std::swap(ptr, o.ptr);
         std::swap(bytes, o.bytes);
     }
+    // room for n bytes, keeping a larger buffer (contents are undefined)
+    void reserve(size_t n) {
+        if (!ptr || bytes < n) alloc(n);
+    }
     template <typename T>
     T* as() const { return static_cast<T*>(ptr); }
     void upload(const void* src, size_t n, hipStream_t s) {

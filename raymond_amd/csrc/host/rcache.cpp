@@ -1,8 +1,6 @@
 // Radiance cache, host side: parameter set-up, the Adam step sequence and the
 // raw-batch entry points.
 #include <cmath>
-#include <cstring>
-#include <limits>
 #include <vector>
 
 #include "rcache_host.h"
@@ -25,27 +23,10 @@ struct InitRng {
     float uniform(float a) { return a * (2.0f * (float)((next() >> 40) * (1.0 / 16777216.0)) - 1.0f); }
 };
 
-// IEEE binary16 bit pattern to float (exact).
-float half_bits_to_float(uint16_t h) {
-    const uint32_t sign = (uint32_t)(h >> 15) << 31;
-    const uint32_t e = (h >> 10) & 0x1fu, m = h & 0x3ffu;
-    float v;
-    if (e == 0u) {
-        v = std::ldexp((float)m, -24);  // zero and subnormals
-    } else if (e == 31u) {
-        v = m ? std::numeric_limits<float>::quiet_NaN() : std::numeric_limits<float>::infinity();
-    } else {
-        v = std::ldexp((float)(m | 0x400u), (int)e - 25);
-    }
-    return sign ? -v : v;
-}
-
-// Feature-major copy of n x k row-major host rows.
-std::vector<float> to_columns(const float* rows, uint32_t n, int k) {
-    std::vector<float> cols((size_t)n * k);
-    for (uint32_t i = 0; i < n; i++)
-        for (int j = 0; j < k; j++) cols[(size_t)j * n + i] = rows[(size_t)i * k + j];
-    return cols;
+// Rows of a raw batch, as the caller has them.
+void stage_rows(DevBuf& buf, const float* rows, size_t floats, hipStream_t s) {
+    buf.reserve(floats * 4);
+    RM_HIP(hipMemcpyAsync(buf.ptr, rows, floats * 4, hipMemcpyHostToDevice, s));
 }
 
 void zero_grads(rm_cache* c, hipStream_t s) {
@@ -212,37 +193,27 @@ void cache_write_params(rm_cache* c, const float* mlp, size_t mlp_count, const f
 void cache_infer_raw(rm_cache* c, const float* features, uint32_t n, float* out) {
     if (n == 0) return;
     hipStream_t s = c->dev->stream;
-    const std::vector<float> cols = to_columns(features, n, kRcFeatureFloats);
-    c->stage_feat.upload(cols.data(), cols.size() * 4, s);
-    c->stage_out.alloc((size_t)n * 3 * 4);
+    stage_rows(c->stage_feat, features, (size_t)n * kRcFeatureFloats, s);
+    c->stage_out.reserve((size_t)n * 3 * 4);
     RcInferArgs a{};
     a.p = cache_params(c);
     a.feat = c->stage_feat.as<float>();
     a.count = n;
-    a.stride = n;
     a.out = c->stage_out.as<float>();
     const uint32_t blocks = std::min<uint32_t>((n + 127) / 128, 4096);
     RM_HIP(launch_rc_infer(a, (int)blocks, s));
-    std::vector<float> res((size_t)n * 3);
-    RM_HIP(hipMemcpyAsync(res.data(), c->stage_out.ptr, res.size() * 4, hipMemcpyDeviceToHost, s));
+    RM_HIP(hipMemcpyAsync(out, c->stage_out.ptr, (size_t)n * 3 * 4, hipMemcpyDeviceToHost, s));
     RM_HIP(hipStreamSynchronize(s));
-    for (uint32_t i = 0; i < n; i++)
-        for (int k = 0; k < 3; k++) out[(size_t)i * 3 + k] = res[(size_t)k * n + i];
 }
 
 static RcSamples stage_samples(rm_cache* c, const float* features, const float* targets, uint32_t n) {
     hipStream_t s = c->dev->stream;
-    const std::vector<float> f = to_columns(features, n, kRcFeatureFloats);
-    const std::vector<float> t = to_columns(targets, n, 3);
-    c->stage_feat.upload(f.data(), f.size() * 4, s);
-    c->stage_target.upload(t.data(), t.size() * 4, s);
+    stage_rows(c->stage_feat, features, (size_t)n * kRcFeatureFloats, s);
+    stage_rows(c->stage_target, targets, (size_t)n * 3, s);
     RcSamples smp{};
     smp.feat = c->stage_feat.as<float>();
     smp.target = c->stage_target.as<float>();
-    smp.stride = n;
     smp.count = n;
-    smp.first = 0;
-    smp.perm_mul = 1;
     return smp;
 }
 
@@ -253,13 +224,14 @@ void cache_gradients_raw(rm_cache* c, const float* features, const float* target
     const RcSamples smp = stage_samples(c, features, targets, n);
     RM_HIP(launch_rc_fill(c->loss.as<float>(), 0.0f, 1, s));
     cache_backward(c, smp, n, s);
+    if (grad_table) RM_HIP(launch_rc_table_grads(c->t_grad.as<uint32_t>(), c->t_master.as<float>(), c->table_floats, s));
+    else RM_HIP(launch_rc_fill(c->t_grad.as<float>(), 0.0f, c->table_floats / 2, s));
     if (grad_mlp) RM_HIP(hipMemcpyAsync(grad_mlp, c->w_grad.ptr, kRcMlpParams * 4, hipMemcpyDeviceToHost, s));
-    std::vector<uint16_t> bits(grad_table ? c->table_floats : 0);
-    if (grad_table) RM_HIP(hipMemcpyAsync(bits.data(), c->t_grad.ptr, c->table_floats * 2, hipMemcpyDeviceToHost, s));
+    RM_HIP(launch_rc_fill(c->w_grad.as<float>(), 0.0f, kRcMlpParams, s));
     if (loss) RM_HIP(hipMemcpyAsync(loss, c->loss.ptr, 4, hipMemcpyDeviceToHost, s));
-    zero_grads(c, s);
+    if (grad_table)
+        RM_HIP(hipMemcpyAsync(grad_table, c->t_master.ptr, c->table_floats * 4, hipMemcpyDeviceToHost, s));
     RM_HIP(hipStreamSynchronize(s));
-    for (size_t i = 0; i < bits.size(); i++) grad_table[i] = half_bits_to_float(bits[i]) / kRcTableGradScale;
 }
 
 void cache_train_raw(rm_cache* c, const float* features, const float* targets, uint32_t n, uint32_t steps,

@@ -10,12 +10,12 @@ struct rm_cache {
     size_t table_floats = 0;
     // FP32 masters, Adam moments, gradients and the FP16 copies the kernels read
     rm::DevBuf t_state;            // Adam records, 8 floats per table pair
-    rm::DevBuf t_master;           // FP32 table staging for parameter reads and writes
+    rm::DevBuf t_master;           // FP32 table staging: parameter reads and writes, gradient reads
     rm::DevBuf t_grad, t_half;
     rm::DevBuf w_master, w_m, w_v, w_grad, w_half;
     rm::DevBuf partial, loss;
     uint32_t partial_waves = 0;
-    // raw-batch staging
+    // raw-batch staging, kept for the next batch
     rm::DevBuf stage_feat, stage_target, stage_out;
     uint64_t steps = 0, samples = 0, queries = 0, records = 0;
     float last_loss = 0.0f;

@@ -194,6 +194,18 @@ __device__ inline void rc_inputs(const RcParams& p, const float* f, int hi, half
     x[5][3] = (_Float16)0.0f;
 }
 
+// Row i of a raw batch: 12 floats, three 16-byte loads.
+__device__ inline void load_row(const float* rows, uint32_t i, bool valid, float* f) {
+    typedef float row4 __attribute__((ext_vector_type(4)));
+    const row4* r = reinterpret_cast<const row4*>(rows + (size_t)i * kRcFeatureFloats);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const row4 v = valid ? r[c] : row4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 4; k++) f[4 * c + k] = v[k];
+    }
+}
+
 struct RcAct {
     half4_t h1[8], h2[8];
     acc16_t y;
@@ -262,8 +274,7 @@ __global__ __launch_bounds__(64 * kInferWaves, 3) void rc_infer_kernel(RcInferAr
                 for (int k = 0; k < 4; k++) f[4 * c + k] = v[k];
             }
         } else {
-#pragma unroll
-            for (int k = 0; k < kRcFeatureFloats; k++) f[k] = valid ? a.feat[(size_t)k * a.stride + i] : 0.0f;
+            load_row(a.feat, i, valid, f);
         }
         half4_t x[6];
         rc_inputs(a.p, f, hi, x);
@@ -287,9 +298,10 @@ __global__ __launch_bounds__(64 * kInferWaves, 3) void rc_infer_kernel(RcInferAr
                 v[3] = 0.0f;
                 reinterpret_cast<row4*>(a.out)[row] = v;
             } else {
-                a.out[i] = act.y[0];
-                a.out[(size_t)count + i] = act.y[1];
-                a.out[2 * (size_t)count + i] = act.y[2];
+                float* o = a.out + 3 * (size_t)i;
+                o[0] = act.y[0];
+                o[1] = act.y[1];
+                o[2] = act.y[2];
             }
         }
     }
@@ -437,18 +449,24 @@ __global__ __launch_bounds__(64 * kTrainWaves) void rc_train_kernel(RcParams p, 
     const uint32_t gwave = blockIdx.x * kTrainWaves + wave;
     const uint32_t j = gwave * 32u + (uint32_t)n;
     const bool valid = j < batch && smp.count > 0;
-    uint32_t rec = 0;
-    if (valid) {
-        if (smp.order) {
+    float f[kRcFeatureFloats];
+    // element c of the sample's target: target[c * t_comp]
+    const float* target = smp.target;
+    uint32_t t_comp = 1u;
+    if (smp.order) {
+        uint32_t rec = 0;
+        if (valid) {
             const uint32_t q = (uint32_t)(((double)j + (double)smp.offset) * (double)smp.count / (double)batch);
             rec = smp.order[q < smp.count ? q : smp.count - 1u];
-        } else {
-            rec = (uint32_t)((((uint64_t)smp.first + j) * smp.perm_mul) % smp.count);
         }
-    }
-    float f[kRcFeatureFloats];
 #pragma unroll
-    for (int k = 0; k < kRcFeatureFloats; k++) f[k] = valid ? smp.feat[(size_t)k * smp.stride + rec] : 0.0f;
+        for (int k = 0; k < kRcFeatureFloats; k++) f[k] = valid ? smp.feat[(size_t)k * smp.stride + rec] : 0.0f;
+        target += rec;
+        t_comp = smp.stride;
+    } else {
+        load_row(smp.feat, j, valid, f);
+        target += 3 * (size_t)j;
+    }
     half4_t x[6];
     rc_inputs(p, f, hi, x);
     RcAct act;
@@ -462,7 +480,7 @@ __global__ __launch_bounds__(64 * kTrainWaves) void rc_train_kernel(RcParams p, 
         float t[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            t[c] = smp.target[(size_t)c * smp.stride + rec];
+            t[c] = target[(size_t)c * t_comp];
             ok = ok && isfinite_(t[c]);
         }
         if (ok) {
@@ -673,6 +691,24 @@ __global__ void rc_table_master_kernel(float* state, float* master, uint32_t* ta
     }
 }
 
+// Table gradients as the caller reads them: FP32, unscaled, from the scaled
+// FP16 sums, which are cleared for the next step.  Four pairs a thread; only
+// pairs that a sample touched are written back.  The host converted them
+// before: a gradients call on 8192 rows with the 2^19 table took 41.6 ms, and
+// takes 6.6 (64 MiB of gradients to the host; this pass moves 100 MB in HBM).
+__global__ void rc_table_grads_kernel(uint32_t* grad_h2, float* out, size_t quads) {
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    const float unscale = 1.0f / kRcTableGradScale;
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < quads; i += stride) {
+        uint4* g = reinterpret_cast<uint4*>(grad_h2) + i;
+        const uint4 w = *g;
+        float4* o = reinterpret_cast<float4*>(out) + 2 * i;
+        o[0] = make_float4(half_lo(w.x) * unscale, half_hi(w.x) * unscale, half_lo(w.y) * unscale, half_hi(w.y) * unscale);
+        o[1] = make_float4(half_lo(w.z) * unscale, half_hi(w.z) * unscale, half_lo(w.w) * unscale, half_hi(w.w) * unscale);
+        if (w.x | w.y | w.z | w.w) *g = make_uint4(0u, 0u, 0u, 0u);
+    }
+}
+
 __global__ void rc_targets_kernel(RcTrainQueue q, const float* slot_radiance, uint32_t c, uint32_t capacity,
                                   float* target) {
     const uint32_t count = c < capacity ? c : capacity;
@@ -730,6 +766,11 @@ hipError_t launch_rc_adam_mlp(const RcAdam& a, hipStream_t s) {
 }
 hipError_t launch_rc_adam_table(const RcAdam& a, hipStream_t s) {
     hipLaunchKernelGGL(rc_adam_table_kernel, dim3(2048), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+hipError_t launch_rc_table_grads(uint32_t* grad_h2, float* out, size_t table_floats, hipStream_t s) {
+    // 2^log2_table_size >= 256 pairs per level: a multiple of four
+    hipLaunchKernelGGL(rc_table_grads_kernel, dim3(2048), dim3(256), 0, s, grad_h2, out, table_floats / 8);
     return hipGetLastError();
 }
 hipError_t launch_rc_targets(const RcTrainQueue& q, const float* slot_radiance, uint32_t count, uint32_t capacity,

@@ -30,15 +30,15 @@ struct RcGrads {
     float* loss;               // sum of per-sample losses (one float)
 };
 
-// Training samples, feature-major: feat[k * stride + i] for feature k.
+// Training samples.  The renderer's records are feature-major
+// (feat[k * stride + i] for feature k) and read through `order`; a raw batch
+// (order null) is the caller's rows, sample j being row j.
 struct RcSamples {
-    const float* feat;         // kRcFeatureFloats x stride
-    const float* target;       // 3 x stride; a NaN target marks an unusable sample
-    uint32_t stride;
+    const float* feat;         // kRcFeatureFloats x stride, or rows
+    const float* target;       // 3 x stride, or rows; a NaN target marks an unusable sample
+    uint32_t stride;           // records: feature-array stride
     uint32_t count;
-    uint32_t first;            // permutation: sample j of the batch is
-    uint32_t perm_mul;         // record ((first + j) * perm_mul) mod count
-    // Spatially sorted records (null: the permutation above): sample j of a
+    // Spatially sorted records: sample j of a
     // batch of b is record order[floor((j + offset) * count / b)], a
     // systematic sample of the sorted records whose consecutive samples, and
     // so the lanes of a wave, lie close together in the scene.
@@ -49,15 +49,14 @@ struct RcSamples {
 // Lookups: either query rows read through a spatial order (the renderer's
 // path), each adding throughput x prediction to its pixel in `image` (plus
 // one sample in alpha) or, without an image, writing its prediction to
-// out[row]; or feature-major raw batches writing 3 x count outputs.
+// out[row]; or raw batches, the caller's rows in and out.
 struct RcInferArgs {
     RcParams p;
     const float* rows;         // kRcQueryFloats per query, or null for a raw batch
     const uint32_t* order;     // rows in spatial order (null: identity)
-    const float* feat;         // raw batch: kRcFeatureFloats x stride, feature-major
+    const float* feat;         // raw batch: kRcFeatureFloats per row
     uint32_t count;
-    uint32_t stride;           // raw batch: feature-array stride
-    float* out;                // rows: 4 floats per row (prediction, 0); raw: 3 x count
+    float* out;                // rows: 4 floats per row (prediction, 0); raw: 3 per row
     float* image;              // rows: add throughput x prediction to the row's pixel here instead of out
 };
 
@@ -103,6 +102,8 @@ hipError_t launch_rc_train(const RcParams& p, const RcSamples& smp, uint32_t bat
 hipError_t launch_rc_reduce(const float* partial, uint32_t waves, float* grad_mlp, hipStream_t s);
 hipError_t launch_rc_adam_mlp(const RcAdam& a, hipStream_t s);
 hipError_t launch_rc_adam_table(const RcAdam& a, hipStream_t s);
+// Table gradients out as unscaled FP32, clearing the FP16 sums.
+hipError_t launch_rc_table_grads(uint32_t* grad_h2, float* out, size_t table_floats, hipStream_t s);
 // Training records -> targets ((radiance at path end - r) / t).
 hipError_t launch_rc_targets(const RcTrainQueue& q, const float* slot_radiance, uint32_t count, uint32_t capacity,
                              float* target, hipStream_t s);
