@@ -233,7 +233,7 @@ int rm_trace_any(rm_scene* scene, const float* rays, uint32_t n, uint32_t* occlu
  * bary are device arrays in the same layouts (rays 16-byte aligned, bary
  * 8-byte aligned) and the call only enqueues work on `stream` (a
  * hipStream_t; null: the device's stream) without synchronising.  The
- * intermediate state lives in a fixed device array of the library (10.5 MB
+ * intermediate state lives in a fixed device array of the library (8.4 MB
  * per GPU, kept until the process ends), so a call takes at most 262144
  * rays (RM_ERROR_INVALID beyond) and calls that overlap on one GPU race.
  * Deep traversal stacks use the scene's spill rows, allocated when the

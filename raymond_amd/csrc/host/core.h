@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <string>
 #include <memory>
+#include <mutex>
 #include <utility>
 #include <vector>
 
@@ -72,6 +73,11 @@ struct DevBuf {
     }
 };
 
+// Device buffers of a raw host batch.
+struct RawBuffers {
+    DevBuf in, out, counter;
+};
+
 struct JitModule {
     hipModule_t module = nullptr;
     hipFunction_t shade = nullptr;
@@ -111,6 +117,9 @@ struct rm_device {
     int any_blocks_per_cu = 1;
     // this device's address of the allocation-free entry point's fixed array
     uint32_t* noalloc_scratch = nullptr;
+    // raw ray batches: buffers kept between calls, held by one at a time
+    std::mutex raw_mutex;
+    rm::RawBuffers raw;
 };
 
 struct rm_scene {

@@ -612,88 +612,90 @@ void scene_build_envmap(rm_scene* s) {
 // ---------------------------------------------------------------------------
 // Raw batch traversal
 
-static void upload_rays_soa(const float* rays, uint32_t n, DevBuf& buf, hipStream_t st, float** f) {
-    std::vector<float> soa((size_t)n * 8);
-    for (uint32_t i = 0; i < n; i++)
-        for (int k = 0; k < 8; k++) soa[(size_t)k * n + i] = rays[(size_t)8 * i + k];
-    buf.upload(soa.data(), soa.size() * 4, st);
-    for (int k = 0; k < 8; k++) f[k] = buf.as<float>() + (size_t)k * n;
+namespace {
+
+// The device buffers of a raw call: the device's own, kept from call to call
+// up to kRawKeep bytes each, or, while another thread uses those, buffers of
+// the call.
+constexpr size_t kRawKeep = (size_t)256 << 20;
+struct RawLease {
+    std::unique_lock<std::mutex> lock;
+    RawBuffers own;
+    RawBuffers* b;
+    explicit RawLease(rm_device* dev) : lock(dev->raw_mutex, std::try_to_lock), b(lock ? &dev->raw : &own) {}
+    ~RawLease() {
+        for (DevBuf* d : {&b->in, &b->out})
+            if (d->bytes > kRawKeep) d->release();
+    }
+};
+
+// The scheduler's counter, cleared; a batch per wave needs none.
+uint32_t* raw_counter(RawBuffers& b, hipStream_t st) {
+    b.counter.reserve(256);
+    RM_HIP(hipMemsetAsync(b.counter.ptr, 0, 256, st));
+    return b.counter.as<uint32_t>();
 }
+
+}  // namespace
 
 void trace_closest_raw(rm_scene* s, const float* rays, uint32_t n, float* t, uint32_t* inst, uint32_t* prim,
                        float* bary) {
     RM_REQUIRE(s->accel_built, "acceleration structure not built");
     if (n == 0) return;
     hipStream_t st = s->dev->stream;
-    DevBuf in, out, cnt;
-    float* f[8];
-    upload_rays_soa(rays, n, in, st, f);
-    out.alloc((size_t)n * 5 * 4);
-    cnt.alloc(sizeof(Counters));
-    RM_HIP(hipMemsetAsync(cnt.ptr, 0, sizeof(Counters), st));
+    RawLease lease(s->dev);
+    RawBuffers& b = *lease.b;
+    const size_t col = (size_t)n * 4;
+    b.in.reserve(col * 8);
+    b.out.reserve(col * 5);
+    RM_HIP(hipMemcpyAsync(b.in.ptr, rays, col * 8, hipMemcpyHostToDevice, st));
+    // pairs first: 8-byte alignment for any n
+    char* o = b.out.as<char>();
     ClosestArgs a{};
     a.nodes = s->d_nodes.as<Bvh8Node>();
     a.tris = s->d_tris.as<BvhTri>();
     a.tlas = s->two_level ? s->d_tlas.as<TlasInstance>() : nullptr;
     a.root2l = s->root2l;
     a.count = n;
-    a.fetch = &cnt.as<Counters>()->it[0].fetch_closest;
-    a.paths.ox = f[0]; a.paths.oy = f[1]; a.paths.oz = f[2];
-    a.paths.dx = f[4]; a.paths.dy = f[5]; a.paths.dz = f[6];
-    a.tmin_arr = f[3];
-    a.tmax_arr = f[7];
-    float* o = out.as<float>();
-    a.hits.t = o;
-    a.hits.inst = reinterpret_cast<uint32_t*>(o + n);
-    a.hits.prim = reinterpret_cast<uint32_t*>(o + 2 * (size_t)n);
-    a.hits.b0 = o + 3 * (size_t)n;
-    a.hits.b1 = o + 4 * (size_t)n;
+    a.fetch = raw_counter(b, st);
+    a.rays = b.in.as<float4>();
+    a.bary = reinterpret_cast<float2*>(o);
+    a.hits.t = reinterpret_cast<float*>(o + 2 * col);
+    a.hits.inst = reinterpret_cast<uint32_t*>(o + 3 * col);
+    a.hits.prim = reinterpret_cast<uint32_t*>(o + 4 * col);
     a.spill = s->d_spill.as<uint2>();
-    a.counters = cnt.as<Counters>();
     const int blocks = s->dev->props.multiProcessorCount * s->dev->trace_blocks_per_cu;
     RM_HIP(launch_trace_closest(a, blocks, false, st));
-    std::vector<float> host((size_t)n * 5);
-    RM_HIP(hipMemcpyAsync(host.data(), out.ptr, host.size() * 4, hipMemcpyDeviceToHost, st));
+    if (t) RM_HIP(hipMemcpyAsync(t, a.hits.t, col, hipMemcpyDeviceToHost, st));
+    if (inst) RM_HIP(hipMemcpyAsync(inst, a.hits.inst, col, hipMemcpyDeviceToHost, st));
+    if (prim) RM_HIP(hipMemcpyAsync(prim, a.hits.prim, col, hipMemcpyDeviceToHost, st));
+    if (bary) RM_HIP(hipMemcpyAsync(bary, a.bary, 2 * col, hipMemcpyDeviceToHost, st));
     RM_HIP(hipStreamSynchronize(st));
-    for (uint32_t i = 0; i < n; i++) {
-        if (t) t[i] = host[i];
-        if (inst) std::memcpy(&inst[i], &host[n + i], 4);
-        if (prim) std::memcpy(&prim[i], &host[2 * (size_t)n + i], 4);
-        if (bary) {
-            bary[2 * i] = host[3 * (size_t)n + i];
-            bary[2 * i + 1] = host[4 * (size_t)n + i];
-        }
-    }
 }
 
 void trace_any_raw(rm_scene* s, const float* rays, uint32_t n, uint32_t* occluded) {
     RM_REQUIRE(s->accel_built, "acceleration structure not built");
     if (n == 0) return;
     hipStream_t st = s->dev->stream;
-    DevBuf in, out, cnt;
-    float* f[8];
-    upload_rays_soa(rays, n, in, st, f);
-    out.alloc((size_t)n * 4);
-    cnt.alloc(sizeof(Counters));
-    RM_HIP(hipMemsetAsync(cnt.ptr, 0, sizeof(Counters), st));
+    RawLease lease(s->dev);
+    RawBuffers& b = *lease.b;
+    const size_t col = (size_t)n * 4;
+    b.in.reserve(col * 8);
+    b.out.reserve(col);
+    RM_HIP(hipMemcpyAsync(b.in.ptr, rays, col * 8, hipMemcpyHostToDevice, st));
     AnyArgs a{};
     a.nodes = s->d_nodes.as<Bvh8Node>();
     a.tris = s->d_tris.as<BvhTri>();
     a.tlas = s->two_level ? s->d_tlas.as<TlasInstance>() : nullptr;
     a.root2l = s->root2l;
     a.count = n;
-    a.fetch = &cnt.as<Counters>()->it[0].fetch_any;
-    a.shadows.ox = f[0]; a.shadows.oy = f[1]; a.shadows.oz = f[2];
-    a.shadows.dx = f[4]; a.shadows.dy = f[5]; a.shadows.dz = f[6];
-    a.tmin_arr = f[3];
-    a.shadows.tmax = f[7];
-    a.image = nullptr;
-    a.occluded = out.as<uint32_t>();
+    a.fetch = raw_counter(b, st);
+    a.rays = b.in.as<float4>();
+    a.occluded = b.out.as<uint32_t>();
     a.spill = s->d_spill.as<uint2>();
-    a.counters = cnt.as<Counters>();
     const int blocks = s->dev->props.multiProcessorCount * s->dev->any_blocks_per_cu;
     RM_HIP(launch_trace_any(a, blocks, false, st));
-    RM_HIP(hipMemcpyAsync(occluded, out.ptr, (size_t)n * 4, hipMemcpyDeviceToHost, st));
+    RM_HIP(hipMemcpyAsync(occluded, b.out.ptr, col, hipMemcpyDeviceToHost, st));
     RM_HIP(hipStreamSynchronize(st));
 }
 

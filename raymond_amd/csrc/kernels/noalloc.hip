@@ -9,11 +9,13 @@
 // when the device is created.  Every call on a GPU shares that copy, so
 // calls that overlap on one GPU race.
 //
-// Layout of `scratch` (32-bit words):
-//   [0, 64)                 persistent-scheduler counter (word 0), cleared
-//                           by a kernel at every call (no memset node)
-//   then 10 arrays of kNoAllocMaxRays words: the rays' origin x/y/z, tmin,
-//   direction x/y/z, tmax, and the hit barycentrics b0, b1
+// The trace kernel reads the caller's rays and writes the caller's hits.
+// `scratch` holds the persistent scheduler's counter, which a batch of more
+// than one 64-ray batch per wave uses and a kernel clears first (no memset
+// node), and a copy of the rays for callers whose hit arrays overlap them.
+// Without the two copies to and from columns that every call made, 100003
+// rays over 82k triangles take 83 us instead of 106; what is left is the
+// longest ray's chain of steps.
 #include <hip/hip_runtime.h>
 
 #include "../host/core.h"
@@ -23,9 +25,7 @@
 namespace rm {
 
 constexpr size_t kNoAllocHeadWords = 64;
-constexpr size_t kNoAllocWords = kNoAllocHeadWords + 10 * (size_t)kNoAllocMaxRays;
-
-static __device__ __align__(256) uint32_t scratch[kNoAllocWords];
+static __device__ __align__(256) uint32_t scratch[kNoAllocHeadWords + 8 * (size_t)kNoAllocMaxRays];
 
 void noalloc_init(rm_device* dev) {
     void* ptr = nullptr;
@@ -34,31 +34,16 @@ void noalloc_init(rm_device* dev) {
     dev->noalloc_scratch = static_cast<uint32_t*>(ptr);
 }
 
-// rays AoS (n x 8) -> SoA columns of the scratch array; clears the counter
-__global__ void noalloc_unpack_kernel(const float* __restrict__ rays, uint32_t n, uint32_t* __restrict__ s) {
+__global__ void noalloc_clear_kernel(uint32_t* s) { s[threadIdx.x] = 0u; }
+
+__global__ void noalloc_copy_kernel(const float4* __restrict__ rays, uint32_t n, float4* __restrict__ copy) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) s[0] = 0u;
-    if (i >= n) return;
-    float* cols = reinterpret_cast<float*>(s + kNoAllocHeadWords);
-    const float4 a = reinterpret_cast<const float4*>(rays)[2 * (size_t)i];
-    const float4 b = reinterpret_cast<const float4*>(rays)[2 * (size_t)i + 1];
-    cols[0 * (size_t)kNoAllocMaxRays + i] = a.x;
-    cols[1 * (size_t)kNoAllocMaxRays + i] = a.y;
-    cols[2 * (size_t)kNoAllocMaxRays + i] = a.z;
-    cols[3 * (size_t)kNoAllocMaxRays + i] = a.w;
-    cols[4 * (size_t)kNoAllocMaxRays + i] = b.x;
-    cols[5 * (size_t)kNoAllocMaxRays + i] = b.y;
-    cols[6 * (size_t)kNoAllocMaxRays + i] = b.z;
-    cols[7 * (size_t)kNoAllocMaxRays + i] = b.w;
+    if (i < 2u * n) copy[i] = rays[i];
 }
 
-// barycentric columns -> the caller's interleaved pairs
-__global__ void noalloc_pack_kernel(const uint32_t* __restrict__ s, uint32_t n, float* __restrict__ bary) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float* cols = reinterpret_cast<const float*>(s + kNoAllocHeadWords);
-    reinterpret_cast<float2*>(bary)[i] =
-        make_float2(cols[8 * (size_t)kNoAllocMaxRays + i], cols[9 * (size_t)kNoAllocMaxRays + i]);
+static bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return x < y + nb && y < x + na;
 }
 
 void trace_closest_noalloc(rm_scene* sc, const float* rays, uint32_t n, float* t, uint32_t* inst, uint32_t* prim,
@@ -72,10 +57,6 @@ void trace_closest_noalloc(rm_scene* sc, const float* rays, uint32_t n, float* t
     RM_REQUIRE(s != nullptr, "allocation-free scratch array not set up on this device");
     if (n == 0) return;
     hipStream_t st = stream ? stream : sc->dev->stream;
-    const uint32_t blocks = (n + 255) / 256;
-    hipLaunchKernelGGL(noalloc_unpack_kernel, dim3(blocks), dim3(256), 0, st, rays, n, s);
-    RM_HIP(hipGetLastError());
-    float* cols = reinterpret_cast<float*>(s + kNoAllocHeadWords);
     ClosestArgs a{};
     a.nodes = sc->d_nodes.as<Bvh8Node>();
     a.tlas = sc->two_level ? sc->d_tlas.as<TlasInstance>() : nullptr;
@@ -83,25 +64,27 @@ void trace_closest_noalloc(rm_scene* sc, const float* rays, uint32_t n, float* t
     a.tris = sc->d_tris.as<BvhTri>();
     a.count = n;
     a.fetch = s;
-    a.paths.ox = cols;
-    a.paths.oy = cols + (size_t)kNoAllocMaxRays;
-    a.paths.oz = cols + 2 * (size_t)kNoAllocMaxRays;
-    a.tmin_arr = cols + 3 * (size_t)kNoAllocMaxRays;
-    a.paths.dx = cols + 4 * (size_t)kNoAllocMaxRays;
-    a.paths.dy = cols + 5 * (size_t)kNoAllocMaxRays;
-    a.paths.dz = cols + 6 * (size_t)kNoAllocMaxRays;
-    a.tmax_arr = cols + 7 * (size_t)kNoAllocMaxRays;
+    a.rays = reinterpret_cast<const float4*>(rays);
+    a.bary = reinterpret_cast<float2*>(bary);
     a.hits.t = t;
     a.hits.inst = inst;
     a.hits.prim = prim;
-    a.hits.b0 = cols + 8 * (size_t)kNoAllocMaxRays;
-    a.hits.b1 = cols + 9 * (size_t)kNoAllocMaxRays;
     a.spill = sc->d_spill.as<uint2>();
     a.counters = nullptr;
+    const size_t nr = (size_t)n * 32, nh = (size_t)n * 4;
+    if (overlap(rays, nr, t, nh) || overlap(rays, nr, inst, nh) || overlap(rays, nr, prim, nh) ||
+        overlap(rays, nr, bary, 2 * nh)) {
+        float4* copy = reinterpret_cast<float4*>(s + kNoAllocHeadWords);
+        hipLaunchKernelGGL(noalloc_copy_kernel, dim3((2 * n + 255) / 256), dim3(256), 0, st, a.rays, n, copy);
+        RM_HIP(hipGetLastError());
+        a.rays = copy;
+    }
     const int tblocks = sc->dev->props.multiProcessorCount * sc->dev->trace_blocks_per_cu;
+    if ((n + kTraceBlock - 1) / kTraceBlock > (uint32_t)trace_closest_blocks(sc->two_level, tblocks)) {
+        hipLaunchKernelGGL(noalloc_clear_kernel, dim3(1), dim3(64), 0, st, s);
+        RM_HIP(hipGetLastError());
+    }
     RM_HIP(launch_trace_closest(a, tblocks, false, st));
-    hipLaunchKernelGGL(noalloc_pack_kernel, dim3(blocks), dim3(256), 0, st, s, n, bary);
-    RM_HIP(hipGetLastError());
 }
 
 }  // namespace rm

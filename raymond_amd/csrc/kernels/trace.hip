@@ -416,20 +416,26 @@ constexpr uint32_t kRefillLanes = RM_REFILL_LANES;
 // are claimed one at a time with an atomic on `counter`.  Waves without a
 // batch of their own exit without touching the counter: device-scope atomics
 // on one address serialise across the XCDs, so a queue of a few thousand
-// rays must not cost an atomic per launched wave.
+// rays must not cost an atomic per launched wave.  A queue of at most one
+// batch per wave is assigned statically and never reads the counter.  (Cutting
+// such a queue into batches of 32, 16 or 8 rays, over more waves, measured
+// 100, 93 and 106 us against 94 for 100003 rays, and no change on renders.)
 struct BatchScheduler {
     uint32_t nb, static_nb, nwaves, b;
     bool dynamic;
     __device__ BatchScheduler(uint32_t count) {
-        nb = (count + (uint32_t)kTraceBlock - 1u) / (uint32_t)kTraceBlock;
-        static_nb = nb - nb / 4u;
         nwaves = gridDim.x;
+        nb = (count + (uint32_t)kTraceBlock - 1u) / (uint32_t)kTraceBlock;
+        static_nb = nb <= nwaves ? nb : nb - nb / 4u;
         b = blockIdx.x;
         dynamic = false;
     }
     // next batch index, or >= nb when done
     __device__ uint32_t next(uint32_t* counter) {
-        if (!dynamic && b >= static_nb) dynamic = true;
+        if (!dynamic && b >= static_nb) {
+            if (static_nb == nb) return nb;
+            dynamic = true;
+        }
         if (dynamic) {
             uint32_t v = 0;
             if (threadIdx.x == 0) v = atomicAdd(counter, 1u);
@@ -492,9 +498,11 @@ struct RayPool {
 };
 
 // Closest hit over a path queue.  Camera paths (depth 0) use the camera's
-// clip range, continuation rays (eps, inf) (intersection.metal:201-202);
-// raw batches bring their own ranges.
-template <bool STATS, bool TWO>
+// clip range, continuation rays (eps, inf) (intersection.metal:201-202).
+// RAW: over the caller's rays, which bring their own ranges; an
+// instantiation of its own, since the branch cost the bounce loop's kernel
+// 1.2% on the sphere field.
+template <bool STATS, bool TWO, bool RAW = false>
 __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWaves) void trace_closest_kernel(ClosestArgs a) {
     __shared__ uint2 lds[kLdsStack * kTraceBlock];
     __shared__ float world[TWO ? 6 * kTraceBlock : 1];
@@ -522,21 +530,25 @@ __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWav
         // idle lanes take the next rays of the wave's batch
         if (pool.refill(active)) {
             i = pool.ray;
-            const vec3 o(q.ox[i], q.oy[i], q.oz[i]);
-            const vec3 d(q.dx[i], q.dy[i], q.dz[i]);
+            vec3 o, d;
             uint32_t root = TWO ? a.root2l : 0u;
-            float near_clip = a.camera.near_clip, far_clip = a.camera.far_clip;
-            if (a.batch.jobs) {
-                const JobInfo& job = a.batch.jobs[job_of_pixel(a.batch.jobs, a.batch.num_jobs, q.pixel[i])];
-                root = job.root;
-                near_clip = job.camera.near_clip;
-                far_clip = job.camera.far_clip;
-            }
             float tmin, tmax;
-            if (a.tmin_arr) {
-                tmin = a.tmin_arr[i];
-                tmax = a.tmax_arr[i];
+            if (RAW) {
+                const float4 r0 = a.rays[2 * (size_t)i], r1 = a.rays[2 * (size_t)i + 1];
+                o = vec3(r0.x, r0.y, r0.z);
+                d = vec3(r1.x, r1.y, r1.z);
+                tmin = r0.w;
+                tmax = r1.w;
             } else {
+                o = vec3(q.ox[i], q.oy[i], q.oz[i]);
+                d = vec3(q.dx[i], q.dy[i], q.dz[i]);
+                float near_clip = a.camera.near_clip, far_clip = a.camera.far_clip;
+                if (a.batch.jobs) {
+                    const JobInfo& job = a.batch.jobs[job_of_pixel(a.batch.jobs, a.batch.num_jobs, q.pixel[i])];
+                    root = job.root;
+                    near_clip = job.camera.near_clip;
+                    far_clip = job.camera.far_clip;
+                }
                 const uint32_t depth = meta_depth(q.meta[i]);
                 // a void path's empty range ends its traversal at the root
                 tmin = depth == 0 ? near_clip : (depth == kVoidDepth ? 1.0f : kEps);
@@ -551,8 +563,12 @@ __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWav
             a.hits.t[i] = s.found ? s.best_t : -1.0f;
             a.hits.prim[i] = s.best_prim;
             a.hits.inst[i] = s.best_inst;
-            a.hits.b0[i] = s.bu / s.bdet;
-            a.hits.b1[i] = s.bv / s.bdet;
+            if (RAW) {
+                a.bary[i] = make_float2(s.bu / s.bdet, s.bv / s.bdet);
+            } else {
+                a.hits.b0[i] = s.bu / s.bdet;
+                a.hits.b1[i] = s.bv / s.bdet;
+            }
             if (STATS) {
                 sn += s.n_nodes;
                 st += s.n_tris;
@@ -644,9 +660,9 @@ __global__ void regenerate_kernel(RegenArgs a) {
 }
 
 // Any-hit over the shadow queue.  With accumulate, an unoccluded ray adds
-// (weight, 1) to its pixel (shadow.metal:6-29); otherwise the occlusion flag
-// is written to `occluded`.
-template <bool STATS, bool TWO>
+// (weight, 1) to its pixel (shadow.metal:6-29).  RAW: over the caller's rays,
+// whose occlusion flags are written to `occluded`.
+template <bool STATS, bool TWO, bool RAW = false>
 __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWaves) void trace_any_kernel(AnyArgs a) {
     __shared__ uint2 lds[kLdsStack * kTraceBlock];
     __shared__ float world[TWO ? 6 * kTraceBlock : 1];
@@ -673,10 +689,19 @@ __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWav
     while (true) {
         if (pool.refill(active)) {
             i = pool.ray;
-            const vec3 o(q.ox[i], q.oy[i], q.oz[i]);
-            const vec3 d(q.dx[i], q.dy[i], q.dz[i]);
-            const float tmin = a.tmin_arr ? a.tmin_arr[i] : kEps;
-            const float tmax = q.tmax[i];
+            vec3 o, d;
+            float tmin = kEps, tmax;
+            if (RAW) {
+                const float4 r0 = a.rays[2 * (size_t)i], r1 = a.rays[2 * (size_t)i + 1];
+                o = vec3(r0.x, r0.y, r0.z);
+                d = vec3(r1.x, r1.y, r1.z);
+                tmin = r0.w;
+                tmax = r1.w;
+            } else {
+                o = vec3(q.ox[i], q.oy[i], q.oz[i]);
+                d = vec3(q.dx[i], q.dy[i], q.dz[i]);
+                tmax = q.tmax[i];
+            }
             uint32_t root = TWO ? a.root2l : 0u;
             if (a.batch.jobs) root = a.batch.jobs[job_of_pixel(a.batch.jobs, a.batch.num_jobs, q.pixel[i])].root;
             s.init(root, o, d, tmin, tmax);
@@ -686,7 +711,7 @@ __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWav
         if (!__any(active)) break;
         if (active && s.step<true, STATS, TWO>(a.nodes, a.tris, a.tlas, stk)) {
             const bool hit = s.found;
-            if (a.image) {
+            if (!RAW) {
                 if (!hit) {
                     float* px = a.image + 4u * (size_t)q.pixel[i];
                     atomicAdd(px + 0, q.wx[i]);
@@ -748,14 +773,18 @@ int two_level_blocks(int blocks, bool any) {
 }
 }  // namespace
 
+int trace_closest_blocks(bool two_level, int blocks) { return two_level ? two_level_blocks(blocks, false) : blocks; }
+
 hipError_t launch_trace_closest(const ClosestArgs& a, int blocks, bool stats, hipStream_t stream) {
     if (a.tlas) {
         blocks = two_level_blocks(blocks, false);
-        if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<true, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+        if (a.rays) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<false, true, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+        else if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<true, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
         else hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<false, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
         return hipGetLastError();
     }
-    if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<true, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+    if (a.rays) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<false, false, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+    else if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<true, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
     else hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_closest_kernel<false, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
     return hipGetLastError();
 }
@@ -763,11 +792,13 @@ hipError_t launch_trace_closest(const ClosestArgs& a, int blocks, bool stats, hi
 hipError_t launch_trace_any(const AnyArgs& a, int blocks, bool stats, hipStream_t stream) {
     if (a.tlas) {
         blocks = two_level_blocks(blocks, true);
-        if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<true, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+        if (a.rays) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<false, true, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+        else if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<true, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
         else hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<false, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
         return hipGetLastError();
     }
-    if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<true, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+    if (a.rays) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<false, false, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+    else if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<true, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
     else hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<false, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
     return hipGetLastError();
 }

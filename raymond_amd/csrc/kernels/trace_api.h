@@ -31,8 +31,10 @@ struct ClosestArgs {
     uint32_t* fetch;            // persistent work counter (zero before launch)
     PathQueue paths;
     HitQueue hits;
-    const float* tmin_arr;      // optional per-ray range (raw batches); else eps / inf
-    const float* tmax_arr;
+    // raw batches: the caller's rays (ox, oy, oz, tmin, dx, dy, dz, tmax)
+    // instead of `paths`, and barycentric pairs instead of hits.b0 / b1
+    const float4* rays;
+    float2* bary;
     uint2* spill;               // (kMaxTraceStack - kLdsStack) x grid threads
     Counters* counters;
     Camera camera;              // clip range of depth-0 paths
@@ -72,9 +74,9 @@ struct AnyArgs {
     const uint32_t* count_ptr;
     uint32_t* fetch;
     ShadowQueue shadows;
-    const float* tmin_arr;      // optional; else eps
-    float* image;               // accumulate unoccluded weights when non-null
-    uint32_t* occluded;         // else write 0/1 per ray
+    const float4* rays;         // raw batches: the caller's rays instead of `shadows`, as in ClosestArgs
+    float* image;               // accumulates unoccluded weights
+    uint32_t* occluded;         // raw batches: 0/1 per ray
     float* slot_radiance;       // radiance cache: unoccluded weights of training paths
     uint2* spill;
     Counters* counters;
@@ -87,6 +89,8 @@ struct AnyArgs {
 
 hipError_t launch_trace_closest(const ClosestArgs& a, int blocks, bool stats, hipStream_t stream);
 hipError_t launch_trace_any(const AnyArgs& a, int blocks, bool stats, hipStream_t stream);
+// Persistent workgroups of a closest-hit launch with `blocks` asked for.
+int trace_closest_blocks(bool two_level, int blocks);
 hipError_t launch_regenerate(const RegenArgs& a, int blocks, hipStream_t stream);
 int trace_blocks_per_cu(bool any);
 
