@@ -58,11 +58,15 @@ struct IterCounters {
     uint32_t appended;       // survivors appended by shade(i-1)
     uint32_t generated;      // camera paths generated before iteration i
     uint32_t shadows;        // shadow rays emitted by shade(i)
-    uint32_t fetch_closest;  // persistent-scheduler counters
-    uint32_t fetch_any;
     uint32_t voids;          // new camera paths without a ray (counted in queue, not traced)
-    uint32_t pad1;
+    uint32_t pad[3];
 };
+
+// Work counters of the persistent trace kernels: one per XCD, each in a cache
+// line of its own (BatchScheduler in kernels/trace.hip).
+constexpr int kFetchParts = 8;
+constexpr int kFetchStride = 32;  // words
+constexpr int kFetchWords = kFetchParts * kFetchStride;
 
 constexpr int kMaxIters = 2048;
 // Material-sort bins: surface materials 0..kSortBins-3 get their own bin
@@ -80,6 +84,9 @@ struct Counters {
     uint32_t cache_queries, train_records;
     // first iteration of the chunk a captured bounce-loop graph is running
     uint32_t iter_base, pad_iter;
+    // work counters of closest (0) and any hit (1) in iteration i: set i % 4,
+    // cleared by the closest-hit kernel of iteration i - 2
+    uint32_t fetch[4][2][kFetchWords];
     // traversal statistics (only written by the statistics variants)
     unsigned long long nodes_closest, tris_closest, nodes_any, tris_any;
 };

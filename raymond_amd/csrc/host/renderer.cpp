@@ -156,11 +156,16 @@ struct StageTimer {
 }  // namespace
 
 // One regenerating stream of `samples` samples per pixel.  Iteration i runs
-// regenerate(i) -> closest(i) -> shade(i) -> shadow(i); queue lengths live in
-// device counters.  The host enqueues chunks of kIterChunk iterations and
-// checks for completion one chunk behind the GPU, so the GPU never waits on
-// the host; a chunk enqueued after the loop drained finds empty queues.
+// regenerate(i) -> closest(i) with shadow(i - 1) -> shade(i); queue lengths
+// live in device counters.  The host enqueues chunks of iterations and checks
+// for completion one chunk behind the GPU, so the GPU never waits on the host;
+// a chunk enqueued after the loop drained finds empty queues.  Paths end by
+// max_depth, so once every camera path has been generated the last possible
+// iteration is known: nothing is enqueued beyond it, and regenerate is left
+// out.  A stream that fits the queue is generated in its first iteration and
+// runs without a single check.
 static constexpr uint32_t kIterChunk = 8;
+static constexpr uint32_t kTailChunk = 4;  // once all paths are generated: fewer empty iterations at the end
 static constexpr uint32_t kCacheStreamMax = 8;
 
 void renderer_set_cache(rm_renderer* r, rm_cache* c, uint32_t mode) {
@@ -288,6 +293,13 @@ struct LoopPollRef {
     char* host;
     size_t slot_bytes;
     hipEvent_t* ready;
+    // after the slots: a stream's counters, copied when its loop has ended
+    IterCounters* iterations() const { return reinterpret_cast<IterCounters*>(host + 2 * slot_bytes); }
+    unsigned long long* traversal() const {
+        return reinterpret_cast<unsigned long long*>(iterations() + kMaxIters);
+    }
+    uint32_t* cache_counts() const { return reinterpret_cast<uint32_t*>(traversal() + 4); }
+    static constexpr size_t kTail = sizeof(IterCounters) * kMaxIters + 4 * sizeof(unsigned long long) + 2 * sizeof(uint32_t);
     IterCounters* probe(int slot) const { return reinterpret_cast<IterCounters*>(host + slot * slot_bytes); }
     uint32_t* done(int slot) const {
         return reinterpret_cast<uint32_t*>(host + slot * slot_bytes + sizeof(IterCounters));
@@ -302,7 +314,7 @@ static LoopPollRef loop_poll(rm_renderer* r, size_t slot_bytes) {
         if (p.host) RM_HIP(hipHostFree(p.host));
         p.host = nullptr;
         p.slot_bytes = 0;
-        RM_HIP(hipHostMalloc(&p.host, 2 * slot_bytes, hipHostMallocDefault));
+        RM_HIP(hipHostMalloc(&p.host, 2 * slot_bytes + LoopPollRef::kTail, hipHostMallocDefault));
         p.slot_bytes = slot_bytes;
     }
     return LoopPollRef{static_cast<char*>(p.host), p.slot_bytes, p.ready};
@@ -322,6 +334,7 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
     const int tbpc = want ? std::min((int)want, dev->trace_blocks_per_cu) : dev->trace_blocks_per_cu;
     const int abpc = want ? std::min((int)want, dev->any_blocks_per_cu) : dev->any_blocks_per_cu;
     const int tblocks = cus * tbpc;
+    const int bblocks = cus * std::min(tbpc, abpc);
     const int ablocks = cus * abpc;
     BatchRun* br = r->batch;
     hipFunction_t shade_fn = br ? s->jit.shade_batch : (r->cache_mode ? s->jit_cache.shade_cache : s->jit.shade);
@@ -416,27 +429,44 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
     aa.counters = cnt;
     if (br) aa.batch = br->view;
 
-    // One iteration: regenerate, closest hit, material sort, shade, shadow
-    // rays.  Directly launched, `it` is the iteration; inside a captured chunk
-    // it is the offset from the device counter iter_base (chunks start at even
-    // iterations, so the queue parity is the offset's).
+    // Separate trace launches when stages are timed or traversal counted.
+    const bool merged = !tm.on && !tstats;
+    // every camera path has been generated by the first iteration, or by a
+    // checked one; paths end before iteration `last` then
+    bool drain = total <= r->capacity;
+    uint32_t last = drain ? r->max_depth : ~0u;
+
+    // One iteration: regenerate, closest hit (with the previous iteration's
+    // shadow rays), material sort, shade.  Directly launched, `it` is the
+    // iteration; inside a captured chunk it is the offset from the device
+    // counter iter_base (chunks start at even iterations, so the queue parity
+    // is the offset's).
     const uint32_t* iter_dev = nullptr;
+    if (cached) {
+        aa.shadows.slot = cache_train ? r->shadow_slot_buf.as<uint32_t>() : nullptr;
+        aa.slot_radiance = cache_train ? r->cv.slot_radiance : nullptr;
+    }
     auto enqueue = [&](uint32_t it) {
         PathQueue& cur = r->q[it & 1];
         PathQueue& next = r->q[(it + 1) & 1];
-        ga.iter = it;
-        ga.iter_dev = iter_dev;
-        ga.paths = cur;
-        ga.slots = slot_arr[it & 1];
-        RM_HIP(launch_regenerate(ga, cus * 4, st));
+        ca.drain = drain && !iter_dev && it > 0;
+        if (!ca.drain) {
+            ga.iter = it;
+            ga.iter_dev = iter_dev;
+            ga.paths = cur;
+            ga.slots = slot_arr[it & 1];
+            RM_HIP(launch_regenerate(ga, cus * 4, st));
+        }
         ca.iter = it;
         ca.iter_dev = iter_dev;
-        ca.count_ptr = iter_dev ? nullptr : &cnt->it[it].queue;
-        ca.fetch = iter_dev ? nullptr : &cnt->it[it].fetch_closest;
         ca.paths = cur;
-        hipEvent_t e = tm.begin();
-        RM_HIP(launch_trace_closest(ca, tblocks, tstats, st));
-        tm.end(e, tm.closest);
+        if (merged) {
+            RM_HIP(launch_trace_both(ca, aa, bblocks, st));
+        } else {
+            hipEvent_t e = tm.begin();
+            RM_HIP(launch_trace_closest(ca, tblocks, tstats, st));
+            tm.end(e, tm.closest);
+        }
         if (sorting) {
             so.iter = it;
             so.iter_dev = iter_dev;
@@ -469,17 +499,13 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
         hipEvent_t es = tm.begin();
         RM_HIP(hipModuleLaunchKernel(shade_fn, sblocks, 1, 1, 256, 1, 1, 0, st, args, nullptr));
         tm.end(es, tm.shade);
-        if (cached) {
-            aa.shadows.slot = cache_train ? r->shadow_slot_buf.as<uint32_t>() : nullptr;
-            aa.slot_radiance = cache_train ? r->cv.slot_radiance : nullptr;
+        if (!merged) {
+            aa.iter = it;
+            aa.iter_dev = iter_dev;
+            hipEvent_t ea = tm.begin();
+            RM_HIP(launch_trace_any(aa, ablocks, tstats, st));
+            tm.end(ea, tm.any);
         }
-        aa.iter = it;
-        aa.iter_dev = iter_dev;
-        aa.count_ptr = iter_dev ? nullptr : &cnt->it[it].shadows;
-        aa.fetch = iter_dev ? nullptr : &cnt->it[it].fetch_any;
-        hipEvent_t ea = tm.begin();
-        RM_HIP(launch_trace_any(aa, ablocks, tstats, st));
-        tm.end(ea, tm.any);
     };
 
     // Captured bounce loop: a chunk of kIterChunk iterations and the advance
@@ -523,33 +549,58 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
             RM_HIP(hipGraphLaunch(chunk_exec, st));
             iter += kIterChunk;
         } else {
-            for (uint32_t c = 0; c < kIterChunk; c++, iter++) enqueue(iter);
+            const uint32_t n = std::min(drain && iter > 0 ? kTailChunk : kIterChunk, last - iter);
+            for (uint32_t c = 0; c < n; c++, iter++) enqueue(iter);
         }
+        chunk_end[slot] = iter;
+        if (iter >= last && !br) return;  // nothing left to check
         RM_HIP(hipMemcpyAsync(lp.probe(slot), &cnt->it[iter], sizeof(IterCounters), hipMemcpyDeviceToHost, st));
         if (br) RM_HIP(hipMemcpyAsync(lp.done(slot), br->view.done, (size_t)njobs * 4, hipMemcpyDeviceToHost, st));
         RM_HIP(hipEventRecord(lp.ready[slot], st));
-        chunk_end[slot] = iter;
     };
-    std::vector<IterCounters> host_it;
     int slot = 0;
     enqueue_chunk(0);
     for (;;) {
+        if (iter >= last) {
+            // the loop ends with what is enqueued; its last shadow rays have
+            // no next iteration to go with
+            if (br) {
+                RM_HIP(hipEventSynchronize(lp.ready[slot]));
+                batch_poll_counts(br, lp.done(slot));
+            }
+            chunk_end[slot] = iter;
+            if (merged) {
+                aa.iter = iter - 1;
+                aa.iter_dev = nullptr;
+                RM_HIP(launch_trace_any(aa, ablocks, false, st));
+            }
+            break;
+        }
         enqueue_chunk(slot ^ 1);  // runs while the host reads the previous chunk's counters
         RM_HIP(hipEventSynchronize(lp.ready[slot]));
         if (br) batch_poll_counts(br, lp.done(slot));
         const IterCounters& probe = *lp.probe(slot);
-        if (probe.generated >= total && probe.appended == 0) break;
+        if (probe.generated >= total) {
+            if (probe.appended == 0) break;
+            // generated before iteration chunk_end[slot]
+            if (!drain) last = chunk_end[slot] - 1 + r->max_depth;
+            drain = true;
+        }
         slot ^= 1;
     }
-    // the chunk after the last one held no work: the stream's statistics and
-    // stage timers end with the chunk that drained it
+    // a chunk after the last one holds no work but the last shadow rays: the
+    // stream's statistics and stage timers end with the chunk that drained it
     iter = chunk_end[slot];
     for (auto* v : {&tm.closest, &tm.sort, &tm.shade, &tm.any})
         if (v->size() > iter) v->resize(iter);
-    uint32_t cache_ctr[2] = {0, 0};  // lookups, training vertices
+    RM_HIP(hipMemcpyAsync(lp.iterations(), cnt->it, iter * sizeof(IterCounters), hipMemcpyDeviceToHost, st));
+    if (tstats)
+        RM_HIP(hipMemcpyAsync(lp.traversal(), &cnt->nodes_closest, 4 * sizeof(unsigned long long),
+                              hipMemcpyDeviceToHost, st));
+    if (cached) RM_HIP(hipMemcpyAsync(lp.cache_counts(), &cnt->cache_queries, 8, hipMemcpyDeviceToHost, st));
+    RM_HIP(hipStreamSynchronize(st));
     if (cached) {
-        RM_HIP(hipMemcpyAsync(cache_ctr, &cnt->cache_queries, 8, hipMemcpyDeviceToHost, st));
-        RM_HIP(hipStreamSynchronize(st));
+        const uint32_t cache_ctr[2] = {lp.cache_counts()[0], lp.cache_counts()[1]};  // lookups, training vertices
         rm_cache* c = r->cache;
         c->queries += cache_ctr[0];
         hipStream_t cs = st;
@@ -632,11 +683,8 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
         }
         RM_HIP(launch_accum_f64(image, r->image64_buf.as<double>(), W * H * 4, st));
     }
-    host_it.resize(iter);
-    RM_HIP(hipMemcpyAsync(host_it.data(), cnt->it, iter * sizeof(IterCounters), hipMemcpyDeviceToHost, st));
-    unsigned long long tstat[4] = {0, 0, 0, 0};
-    RM_HIP(hipMemcpyAsync(tstat, &cnt->nodes_closest, sizeof(tstat), hipMemcpyDeviceToHost, st));
-    RM_HIP(hipStreamSynchronize(st));
+    if ((cached && !overlap) || r->u.accumulate_f64) RM_HIP(hipStreamSynchronize(st));
+    const IterCounters* host_it = lp.iterations();
     if (cached && tm.on) r->cache->ms_infer += StageTimer::sum(t_infer);
     r->frame_index += samples;
     if (stats) {
@@ -659,10 +707,13 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
             stats->ms_sort += StageTimer::sum(tm.sort);
             stats->ms_trace_any += StageTimer::sum(tm.any);
         }
-        stats->nodes_closest += tstat[0];
-        stats->tris_closest += tstat[1];
-        stats->nodes_any += tstat[2];
-        stats->tris_any += tstat[3];
+        if (tstats) {
+            const unsigned long long* t = lp.traversal();
+            stats->nodes_closest += t[0];
+            stats->tris_closest += t[1];
+            stats->nodes_any += t[2];
+            stats->tris_any += t[3];
+        }
     }
 }
 

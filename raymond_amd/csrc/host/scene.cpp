@@ -629,10 +629,10 @@ struct RawLease {
     }
 };
 
-// The scheduler's counter, cleared; a batch per wave needs none.
+// The scheduler's work counters, cleared.
 uint32_t* raw_counter(RawBuffers& b, hipStream_t st) {
-    b.counter.reserve(256);
-    RM_HIP(hipMemsetAsync(b.counter.ptr, 0, 256, st));
+    b.counter.reserve(kFetchWords * 4);
+    RM_HIP(hipMemsetAsync(b.counter.ptr, 0, kFetchWords * 4, st));
     return b.counter.as<uint32_t>();
 }
 

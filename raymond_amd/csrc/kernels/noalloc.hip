@@ -10,7 +10,7 @@
 // calls that overlap on one GPU race.
 //
 // The trace kernel reads the caller's rays and writes the caller's hits.
-// `scratch` holds the persistent scheduler's counter, which a batch of more
+// `scratch` holds the persistent scheduler's counters, which a batch of more
 // than one 64-ray batch per wave uses and a kernel clears first (no memset
 // node), and a copy of the rays for callers whose hit arrays overlap them.
 // Without the two copies to and from columns that every call made, 100003
@@ -24,7 +24,7 @@
 
 namespace rm {
 
-constexpr size_t kNoAllocHeadWords = 64;
+constexpr size_t kNoAllocHeadWords = kFetchWords;
 static __device__ __align__(256) uint32_t scratch[kNoAllocHeadWords + 8 * (size_t)kNoAllocMaxRays];
 
 void noalloc_init(rm_device* dev) {
@@ -81,7 +81,7 @@ void trace_closest_noalloc(rm_scene* sc, const float* rays, uint32_t n, float* t
     }
     const int tblocks = sc->dev->props.multiProcessorCount * sc->dev->trace_blocks_per_cu;
     if ((n + kTraceBlock - 1) / kTraceBlock > (uint32_t)trace_closest_blocks(sc->two_level, tblocks)) {
-        hipLaunchKernelGGL(noalloc_clear_kernel, dim3(1), dim3(64), 0, st, s);
+        hipLaunchKernelGGL(noalloc_clear_kernel, dim3(1), dim3(kFetchWords), 0, st, s);
         RM_HIP(hipGetLastError());
     }
     RM_HIP(launch_trace_closest(a, tblocks, false, st));

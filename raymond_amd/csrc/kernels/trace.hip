@@ -403,6 +403,8 @@ constexpr int kTraceMinWaves = RM_TRACE_MIN_WAVES;
 #define RM_TWO_LEVEL_MIN_WAVES 5
 #endif
 constexpr int kTwoLevelMinWaves = RM_TWO_LEVEL_MIN_WAVES;
+// Both traversals in one kernel are held to the separate kernels' 5 waves.
+constexpr int kBothMinWaves = 5;
 
 // Lanes are refilled once at least this many of a wave's 64 are idle
 // (with two leaf slots, 4, 12 and 16 measured within 1% of 8).
@@ -411,35 +413,47 @@ constexpr int kTwoLevelMinWaves = RM_TWO_LEVEL_MIN_WAVES;
 #endif
 constexpr uint32_t kRefillLanes = RM_REFILL_LANES;
 
-// Batch scheduler of the persistent waves.  The first 3/4 of the 64-ray
+// Batch scheduler of the persistent waves.  The first 2/5 of the 64-ray
 // batches are assigned statically (wave w takes w, w + nwaves, ...); the rest
-// are claimed one at a time with an atomic on `counter`.  Waves without a
-// batch of their own exit without touching the counter: device-scope atomics
-// on one address serialise across the XCDs, so a queue of a few thousand
-// rays must not cost an atomic per launched wave.  A queue of at most one
-// batch per wave is assigned statically and never reads the counter.  (Cutting
+// are claimed one at a time with an atomic.  Device-scope atomics on one
+// address serialise across the XCDs (about 10 ns each): with one counter, the
+// claims of a quarter of the batches bounded the closest-hit kernel on small
+// trees (Cornell box, 28.7M rays in 8 launches: 1.97 ms).  So there is a
+// counter per workgroup index mod 8, which is the XCD, in a cache line of its
+// own, and part x claims batches x, x + 8, ... of the rest: 1.21 ms.  Claims
+// are then cheap enough to leave more to them.  Shares claimed of 10, 25, 40,
+// 60, 80 and 100% measured (ms per pass) 29.5, 28.3, 27.0, 26.1-27.0, 26.0
+// and 26.0 on the 5.2M-triangle sphere field, 21.0, 20.3, 19.7, 18.0, 17.8 and
+// 17.8 on the instanced field, 4.94, 4.88, 4.82, 4.80, 4.87 and 4.93 on the
+// Cornell box.  Waves without a batch
+// of their own exit without touching a counter, and a queue of at most one
+// batch per wave is assigned statically and never reads one.  (Cutting
 // such a queue into batches of 32, 16 or 8 rays, over more waves, measured
 // 100, 93 and 106 us against 94 for 100003 rays, and no change on renders.)
+constexpr uint32_t kClaimedPercent = 60;
 struct BatchScheduler {
     uint32_t nb, static_nb, nwaves, b;
     bool dynamic;
-    __device__ BatchScheduler(uint32_t count) {
+    // `first`: the wave's place in the assignment (its block, or a rotation)
+    __device__ BatchScheduler(uint32_t count, uint32_t first) {
         nwaves = gridDim.x;
         nb = (count + (uint32_t)kTraceBlock - 1u) / (uint32_t)kTraceBlock;
-        static_nb = nb <= nwaves ? nb : nb - nb / 4u;
-        b = blockIdx.x;
+        static_nb = nb <= nwaves ? nb : nb - (uint32_t)((uint64_t)nb * kClaimedPercent / 100u);
+        b = first;
         dynamic = false;
     }
     // next batch index, or >= nb when done
-    __device__ uint32_t next(uint32_t* counter) {
+    __device__ uint32_t next(uint32_t* counters) {
         if (!dynamic && b >= static_nb) {
             if (static_nb == nb) return nb;
             dynamic = true;
         }
         if (dynamic) {
+            const uint32_t parts = nwaves < (uint32_t)kFetchParts ? nwaves : (uint32_t)kFetchParts;
+            const uint32_t part = blockIdx.x % parts;
             uint32_t v = 0;
-            if (threadIdx.x == 0) v = atomicAdd(counter, 1u);
-            b = static_nb + __shfl(v, 0);
+            if (threadIdx.x == 0) v = atomicAdd(counters + part * (uint32_t)kFetchStride, 1u);
+            b = static_nb + (uint32_t)__builtin_amdgcn_readfirstlane((int)v) * parts + part;
         }
         const uint32_t cur = b;
         if (!dynamic) b += nwaves;
@@ -497,29 +511,42 @@ struct RayPool {
     }
 };
 
+// A wave's stack rows: a column per lane in `lds` and in the spill array.
+template <bool TWO>
+__device__ inline StackRef wave_stack(uint2* lds, float* world, uint2* spill) {
+    const uint32_t lane = threadIdx.x;
+    return StackRef{(lds_u64*)(lds + lane), (global_u64*)(spill + blockIdx.x * kTraceBlock + lane),
+                    gridDim.x * kTraceBlock, (lds_f32*)(world + (TWO ? lane : 0u))};
+}
+
+// Paths of an iteration's queue.  Once every camera path has been generated
+// no regenerate kernel runs, and the queue is the survivors: the trace kernel
+// then records its length for the kernels after it.
+__device__ inline uint32_t queue_length(const ClosestArgs& a, uint32_t it) {
+    IterCounters& ic = a.counters->it[it];
+    // the work counters of iteration it + 2 (last used by it - 2)
+    if (blockIdx.x == 0 && threadIdx.x < 2u * (uint32_t)kFetchParts)
+        a.counters->fetch[(it + 2u) & 3u][threadIdx.x / (uint32_t)kFetchParts]
+                         [threadIdx.x % (uint32_t)kFetchParts * (uint32_t)kFetchStride] = 0u;
+    if (!a.drain) return ic.queue;
+    const uint32_t n = ic.appended;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ic.queue = n;
+        a.counters->it[it + 1].generated = ic.generated;
+    }
+    return n;
+}
+
 // Closest hit over a path queue.  Camera paths (depth 0) use the camera's
 // clip range, continuation rays (eps, inf) (intersection.metal:201-202).
 // RAW: over the caller's rays, which bring their own ranges; an
 // instantiation of its own, since the branch cost the bounce loop's kernel
 // 1.2% on the sphere field.
-template <bool STATS, bool TWO, bool RAW = false>
-__global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWaves) void trace_closest_kernel(ClosestArgs a) {
-    __shared__ uint2 lds[kLdsStack * kTraceBlock];
-    __shared__ float world[TWO ? 6 * kTraceBlock : 1];
-    const uint32_t lane = threadIdx.x;
-    const uint32_t gtid = blockIdx.x * kTraceBlock + lane;
-    StackRef stk{(lds_u64*)(lds + lane), (global_u64*)(a.spill + gtid), gridDim.x * kTraceBlock,
-                 (lds_f32*)(world + (TWO ? lane : 0u))};
-    const uint32_t* count_ptr = a.count_ptr;
-    uint32_t* fetch = a.fetch;
-    if (a.iter_dev) {
-        IterCounters& ic = a.counters->it[iteration_of(a.iter_dev, a.iter)];
-        count_ptr = &ic.queue;
-        fetch = &ic.fetch_closest;
-    }
-    const uint32_t count = count_ptr ? *count_ptr : a.count;
+template <bool STATS, bool TWO, bool RAW>
+__device__ inline __attribute__((always_inline)) void closest_rays(const ClosestArgs& a, const StackRef& stk,
+                                                                   uint32_t count, uint32_t* fetch) {
     unsigned long long sn = 0, st = 0;
-    BatchScheduler sched(count);
+    BatchScheduler sched(count, blockIdx.x);
     if (blockIdx.x >= sched.nb) return;
     const PathQueue& q = a.paths;
     RayState s;
@@ -579,6 +606,19 @@ __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWav
     if (STATS) {
         atomicAdd(&a.counters->nodes_closest, sn);
         atomicAdd(&a.counters->tris_closest, st);
+    }
+}
+
+template <bool STATS, bool TWO, bool RAW = false>
+__global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWaves) void trace_closest_kernel(ClosestArgs a) {
+    __shared__ uint2 lds[kLdsStack * kTraceBlock];
+    __shared__ float world[TWO ? 6 * kTraceBlock : 1];
+    const StackRef stk = wave_stack<TWO>(lds, world, a.spill);
+    if (RAW) {
+        closest_rays<STATS, TWO, RAW>(a, stk, a.count, a.fetch);
+    } else {
+        const uint32_t it = iteration_of(a.iter_dev, a.iter);
+        closest_rays<STATS, TWO, RAW>(a, stk, queue_length(a, it), a.counters->fetch[it & 3u][0]);
     }
 }
 
@@ -659,28 +699,16 @@ __global__ void regenerate_kernel(RegenArgs a) {
     }
 }
 
-// Any-hit over the shadow queue.  With accumulate, an unoccluded ray adds
-// (weight, 1) to its pixel (shadow.metal:6-29).  RAW: over the caller's rays,
-// whose occlusion flags are written to `occluded`.
-template <bool STATS, bool TWO, bool RAW = false>
-__global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWaves) void trace_any_kernel(AnyArgs a) {
-    __shared__ uint2 lds[kLdsStack * kTraceBlock];
-    __shared__ float world[TWO ? 6 * kTraceBlock : 1];
-    const uint32_t lane = threadIdx.x;
-    const uint32_t gtid = blockIdx.x * kTraceBlock + lane;
-    StackRef stk{(lds_u64*)(lds + lane), (global_u64*)(a.spill + gtid), gridDim.x * kTraceBlock,
-                 (lds_f32*)(world + (TWO ? lane : 0u))};
-    const uint32_t* count_ptr = a.count_ptr;
-    uint32_t* fetch = a.fetch;
-    if (a.iter_dev) {
-        IterCounters& ic = a.counters->it[iteration_of(a.iter_dev, a.iter)];
-        count_ptr = &ic.shadows;
-        fetch = &ic.fetch_any;
-    }
-    const uint32_t count = count_ptr ? *count_ptr : a.count;
+// Any-hit over the shadow queue.  An unoccluded ray adds (weight, 1) to its
+// pixel (shadow.metal:6-29).  RAW: over the caller's rays, whose occlusion
+// flags are written to `occluded`.  `first` is the wave's place in the
+// assignment of batches.
+template <bool STATS, bool TWO, bool RAW>
+__device__ inline __attribute__((always_inline)) void any_rays(const AnyArgs& a, const StackRef& stk, uint32_t count,
+                                                               uint32_t* fetch, uint32_t first) {
     unsigned long long sn = 0, st = 0;
-    BatchScheduler sched(count);
-    if (blockIdx.x >= sched.nb) return;
+    BatchScheduler sched(count, first);
+    if (first >= sched.nb) return;
     const ShadowQueue& q = a.shadows;
     RayState s;
     bool active = false;
@@ -743,6 +771,38 @@ __global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWav
     }
 }
 
+template <bool STATS, bool TWO, bool RAW = false>
+__global__ __launch_bounds__(kTraceBlock, TWO ? kTwoLevelMinWaves : kTraceMinWaves) void trace_any_kernel(AnyArgs a) {
+    __shared__ uint2 lds[kLdsStack * kTraceBlock];
+    __shared__ float world[TWO ? 6 * kTraceBlock : 1];
+    const StackRef stk = wave_stack<TWO>(lds, world, a.spill);
+    if (RAW) {
+        any_rays<STATS, TWO, RAW>(a, stk, a.count, a.fetch, blockIdx.x);
+    } else {
+        const uint32_t it = iteration_of(a.iter_dev, a.iter);
+        any_rays<STATS, TWO, RAW>(a, stk, a.counters->it[it].shadows, a.counters->fetch[it & 3u][1], blockIdx.x);
+    }
+}
+
+// Closest hits of iteration i and shadow rays of iteration i - 1, which do not
+// depend on each other, in one launch: a wave that runs out of paths goes on
+// with shadow rays, so the longest rays of one kind overlap work of the other,
+// and a bounce has one launch fewer.  With few paths, the waves without one
+// take the first shadow batches.
+template <bool TWO>
+__global__ __launch_bounds__(kTraceBlock, kBothMinWaves) void trace_both_kernel(ClosestArgs c, AnyArgs a) {
+    __shared__ uint2 lds[kLdsStack * kTraceBlock];
+    __shared__ float world[TWO ? 6 * kTraceBlock : 1];
+    const StackRef stk = wave_stack<TWO>(lds, world, c.spill);
+    const uint32_t it = iteration_of(c.iter_dev, c.iter);
+    const uint32_t paths = queue_length(c, it);
+    const uint32_t shadows = it ? c.counters->it[it - 1u].shadows : 0u;
+    closest_rays<false, TWO, false>(c, stk, paths, c.counters->fetch[it & 3u][0]);
+    const uint32_t busy = (paths + (uint32_t)kTraceBlock - 1u) / (uint32_t)kTraceBlock;
+    const uint32_t first = busy < gridDim.x ? (blockIdx.x + gridDim.x - busy) % gridDim.x : blockIdx.x;
+    any_rays<false, TWO, false>(a, stk, shadows, c.counters->fetch[(it + 3u) & 3u][1], first);
+}
+
 }  // namespace rm
 
 // ---------------------------------------------------------------------------
@@ -800,6 +860,12 @@ hipError_t launch_trace_any(const AnyArgs& a, int blocks, bool stats, hipStream_
     if (a.rays) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<false, false, true>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
     else if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<true, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
     else hipLaunchKernelGGL(HIP_KERNEL_NAME(trace_any_kernel<false, false>), dim3(blocks), dim3(kTraceBlock), 0, stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_trace_both(const ClosestArgs& c, const AnyArgs& a, int blocks, hipStream_t stream) {
+    if (c.tlas) hipLaunchKernelGGL(trace_both_kernel<true>, dim3(blocks), dim3(kTraceBlock), 0, stream, c, a);
+    else hipLaunchKernelGGL(trace_both_kernel<false>, dim3(blocks), dim3(kTraceBlock), 0, stream, c, a);
     return hipGetLastError();
 }
 

@@ -26,9 +26,8 @@ constexpr int kLdsStack = RM_LDS_STACK;
 struct ClosestArgs {
     const Bvh8Node* nodes;
     const BvhTri* tris;
-    uint32_t count;             // used when count_ptr is null
-    const uint32_t* count_ptr;  // device queue length
-    uint32_t* fetch;            // persistent work counter (zero before launch)
+    uint32_t count;             // raw batches: rays
+    uint32_t* fetch;            // raw batches: kFetchWords work counters (zero before launch)
     PathQueue paths;
     HitQueue hits;
     // raw batches: the caller's rays (ox, oy, oz, tmin, dx, dy, dz, tmax)
@@ -39,9 +38,10 @@ struct ClosestArgs {
     Counters* counters;
     Camera camera;              // clip range of depth-0 paths
     BatchView batch;            // batched jobs (jobs null: one scene, root 0)
-    // captured bounce loops: count and fetch come from counters->it[iteration_of(iter_dev, iter)]
+    // bounce loops: count and fetch come from the counters of iteration_of(iter_dev, iter)
     const uint32_t* iter_dev;
     uint32_t iter;
+    uint32_t drain;             // no regenerate kernel ran for this iteration (queue_length)
     // two-level scenes: instance records of the top-level tree (null: flat)
     const TlasInstance* tlas;
     uint32_t root2l;
@@ -70,9 +70,8 @@ struct RegenArgs {
 struct AnyArgs {
     const Bvh8Node* nodes;
     const BvhTri* tris;
-    uint32_t count;
-    const uint32_t* count_ptr;
-    uint32_t* fetch;
+    uint32_t count;             // raw batches: rays
+    uint32_t* fetch;            // raw batches: work counters
     ShadowQueue shadows;
     const float4* rays;         // raw batches: the caller's rays instead of `shadows`, as in ClosestArgs
     float* image;               // accumulates unoccluded weights
@@ -81,7 +80,7 @@ struct AnyArgs {
     uint2* spill;
     Counters* counters;
     BatchView batch;
-    const uint32_t* iter_dev;   // captured bounce loops, as in ClosestArgs
+    const uint32_t* iter_dev;   // bounce loops, as in ClosestArgs
     uint32_t iter;
     const TlasInstance* tlas;   // two-level scenes, as in ClosestArgs
     uint32_t root2l;
@@ -89,6 +88,8 @@ struct AnyArgs {
 
 hipError_t launch_trace_closest(const ClosestArgs& a, int blocks, bool stats, hipStream_t stream);
 hipError_t launch_trace_any(const AnyArgs& a, int blocks, bool stats, hipStream_t stream);
+// Closest hits of c's iteration and the shadow rays of the one before it.
+hipError_t launch_trace_both(const ClosestArgs& c, const AnyArgs& a, int blocks, hipStream_t stream);
 // Persistent workgroups of a closest-hit launch with `blocks` asked for.
 int trace_closest_blocks(bool two_level, int blocks);
 hipError_t launch_regenerate(const RegenArgs& a, int blocks, hipStream_t stream);
