@@ -7,10 +7,10 @@
 //
 // Design:
 //  * persistent waves over the device-resident queue length (no host
-//    round-trip): most 64-ray batches are assigned statically, the tail is
-//    claimed dynamically through a per-depth counter (BatchScheduler);
+//    round-trip): part of the 64-ray batches are assigned statically, the
+//    others are claimed through one counter per XCD (BatchScheduler);
 //  * compressed BVH8 (80-byte nodes, five 16-byte loads, 8-bit child boxes)
-//    with ordered internal-child visits by ray octant;
+//    visiting the nearest internal child hit first (closest hit);
 //  * traversal stack: the bottom kLdsStack entries per lane in LDS (column
 //    per lane), deeper entries spill to a per-thread global array.
 #include <hip/hip_runtime.h>
@@ -37,6 +37,13 @@ __device__ inline float plane_q(const half2v (&h)[4], int c) { return (float)h[c
 __device__ inline uint32_t byte_of(uint32_t lo, uint32_t hi, int c) {
     const uint32_t w = c < 4 ? lo : hi;
     return (w >> (8 * (c & 3))) & 0xffu;
+}
+
+// the middle of three (the compiler forms v_med3 only from longer patterns)
+__device__ inline int med3(int a, int b, int c) {
+    int d;
+    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
 }
 
 // Stack entries as 64-bit words behind pointers typed by address space, so
@@ -114,15 +121,16 @@ constexpr int kHeldShareAny = RM_HELD_SHARE_ANY;
 
 // Traversal state of one lane's ray.  It persists across steps, so a lane
 // whose ray has finished takes a new one while the rest of the wave goes on.
+constexpr uint32_t kNoNode = 0xffffffffu;
+
 struct RayState {
     vec3 o, inv;
     RayShear sh;
-    int oct;
     float tmin, tmax, best_t;
     uint32_t best_inst, best_prim;
     float bu, bv, bdet;  // closest hit's scaled barycentrics and their sum
     bool found;
-    uint2 cur;  // node group: child base, (remaining child hits << 24) | internal mask
+    uint32_t next;  // node to visit, or kNoNode
     uint2 tg;   // postponed leaf triangles: base, mask (top level of a two-level tree: instances)
     uint2 tg2;  // a second postponed leaf set (kLeafSlots == 2)
     int sp;
@@ -136,7 +144,6 @@ struct RayState {
         o = org;
         inv = safe_inv_dir(d);
         sh = make_shear(d);
-        oct = dir_octant(d);
     }
 
     __device__ void init(uint32_t root, vec3 org, vec3 d, float t0, float t1) {
@@ -144,8 +151,7 @@ struct RayState {
         inst = 0;
         top = true;
         marker_sp = -1;
-        // a one-child pseudo node whose only child is the root
-        cur = make_uint2(root, (1u << (24 + oct)) | 1u);
+        next = root;
         sp = 0;
         tmin = t0;
         tmax = t1;
@@ -162,10 +168,16 @@ struct RayState {
         n_tris = 0;
     }
 
+    // Whether a group's bound lies beyond the closest hit so far (a marker's
+    // bound is zero).
+    __device__ bool beyond(uint2 e) const {
+        return __uint_as_float((e.y << 8) & 0x7fff0000u) > fmaxf(best_t * kBoxSlack, 0.0f);
+    }
+
     // Two-level trees: enters the next instance of the top-level leaf set in
-    // tg.  The top-level group (if it has hits left) and a marker entry with
-    // the set's other instances go on the stack; popping the marker returns
-    // to the world ray.  The ray is mapped affinely into the instance's
+    // tg.  A marker entry with the set's other instances goes on the stack
+    // (above the top-level group, which the node step pushed whole); popping
+    // the marker returns to the world ray.  The ray is mapped affinely into the instance's
     // object space without renormalising the direction, so t is the same
     // parameter on both sides, and the shape's tree is visited from its root.
     __device__ void enter(const TlasInstance* __restrict__ insts, const StackRef& stk) {
@@ -173,10 +185,6 @@ struct RayState {
         tg.y &= tg.y - 1u;
         const uint4* ip = reinterpret_cast<const uint4*>(insts + tg.x + (uint32_t)b);
         const uint4 r0 = ip[0], r1 = ip[1], r2 = ip[2], r3 = ip[3];
-        if (cur.y & 0xff000000u) {
-            stk.store(sp, cur);
-            sp++;
-        }
         stk.store(sp, make_uint2(tg.x, kMarker2l | tg.y));
         marker_sp = sp;
         sp++;
@@ -191,7 +199,7 @@ struct RayState {
         set_ray(tlas_point(ti, stk.world_o()), tlas_vector(ti, stk.world_d()));
         inst = r3.y;
         top = false;
-        cur = make_uint2(r3.x, (1u << (24 + oct)) | 1u);
+        next = r3.x;
         tg = make_uint2(0u, 0u);
     }
 
@@ -216,9 +224,9 @@ struct RayState {
         constexpr bool kTwoSlots = kLeafSlots > 1;
         const bool to_enter = TWO && top && tg.y != 0u;
         const bool has_tris = !to_enter && tg.y != 0u;
-        const bool node_work = (cur.y & 0xff000000u) || sp > 0;
+        const bool node_work = next != kNoNode || sp > 0;
         bool can_node = !to_enter && node_work && (kTwoSlots ? tg2.y == 0u : !has_tris);
-        if (TWO && kTwoSlots && has_tris && !(cur.y & 0xff000000u) && sp - 1 == marker_sp) can_node = false;
+        if (TWO && kTwoSlots && has_tris && next == kNoNode && sp - 1 == marker_sp) can_node = false;
         const unsigned long long held = __ballot((has_tris || to_enter) && !can_node);
         if (__popcll(held) * (ANY ? kHeldShareAny : kHeldShare) >= __popcll(__ballot(true)) ||
             __ballot(can_node) == 0ull) {
@@ -235,11 +243,26 @@ struct RayState {
             return ended || (!node_work && tg.y == 0u);
         }
         if (!can_node) return false;
-        if (!(cur.y & 0xff000000u)) {
-            if (sp == 0) return true;
-            sp--;
-            const uint2 e = stk.load(sp);
+        if (next == kNoNode) {
+            // The top group: its first child in slot order, the others stay on
+            // the stack.  A group beyond the closest hit is dropped; in a flat
+            // tree the lane then waits for the next step, in a two-level one
+            // it goes on to the group below (1080p, execute, ms: sphere field
+            // waiting 24.90, going on 25.23; instanced field 18.13 against
+            // 17.78).
+            uint2 e;
+            do {
+                if (TWO && sp == 0) return false;  // ends in the next triangle phase
+                sp--;
+                e = stk.load(sp);
+                if (!ANY && !TWO && beyond(e)) return false;
+            } while (!ANY && TWO && beyond(e));
             if (TWO && (e.y & kMarker2l)) {
+                // pending triangles belong to the instance's ray
+                if (kTwoSlots && has_tris) {
+                    sp++;
+                    return false;
+                }
                 // back in the world: the set's other instances, then the
                 // top-level groups below the marker (entering the next
                 // instance maps the ray again, so the world ray is needed only
@@ -248,20 +271,18 @@ struct RayState {
                 if (tg.y == 0u) set_ray(stk.world_o(), stk.world_d());
                 top = true;
                 marker_sp = -1;
-                cur = make_uint2(0u, 0u);
                 return false;
             }
-            cur = e;  // pushed groups always hold a hit child
+            const uint32_t hits = e.y >> 24;
+            const uint32_t rest = hits & (hits - 1u);
+            next = e.x + __builtin_popcount(e.y & ((hits ^ rest) - 1u) & 0xffu);
+            if (rest) {
+                stk.store(sp, make_uint2(e.x, (e.y & 0xffffffu) | (rest << 24)));
+                sp++;
+            }
         }
-        const uint32_t hits = cur.y >> 24;
-        const int k = __builtin_ctz(hits);
-        cur.y &= ~(1u << (24 + k));
-        const int slot = k ^ oct;
-        const uint32_t node_idx = cur.x + __builtin_popcount(cur.y & 0xffu & ((1u << slot) - 1u));
-        if (cur.y & 0xff000000u) {
-            stk.store(sp, cur);
-            sp++;
-        }
+        const uint32_t node_idx = next;
+        next = kNoNode;
         const uint4* np = reinterpret_cast<const uint4*>(nodes + node_idx);
         const uint4 q0 = np[0], q1 = np[1], q2 = np[2], q3 = np[3], q4 = np[4];
         if (STATS) n_nodes++;
@@ -271,9 +292,9 @@ struct RayState {
         // (exact) and B = (p - o) * inv, one FMA per plane.  The byte q
         // enters as the half 1024 + q (two per v_perm, exact), which
         // v_fma_mix_f32 multiplies in f32, so the offset becomes
-        // B' = (B -+ E) - 1024 A.  With u = 2^-24 the computed plane is within
-        // u (1534 |A| + 6 |B|) of its exact t, (q s + p - o) / d, to first
-        // order, so moving B outward by E = 16u (|B| + 255 |A|) leaves every
+        // B' = (B - 1024 A) -+ E.  With u = 2^-24 the computed plane is within
+        // u (2558 |A| + 7 |B|) of its exact t, (q s + p - o) / d, to first
+        // order, so moving B outward by E = 20u (|B| + 255 |A|) leaves every
         // near plane before and every far plane after the exact one, with a
         // margin of nearly 10u (|B| + 255 |A|) >= 10u |t| for the triangle
         // test's own rounding (best_t keeps the relative slack on top).  A
@@ -284,9 +305,10 @@ struct RayState {
         auto axis = [](float p, uint32_t ebits, float o, float inv, float& A, float& Bn, float& Bf) {
             A = exp_scale((uint8_t)ebits) * inv;
             const float B = (p - o) * inv;
-            const float E = 9.53674316e-7f * (fabsf(B) + 255.0f * fabsf(A));
-            Bn = __builtin_fmaf(-1024.0f, A, B - E);
-            Bf = __builtin_fmaf(-1024.0f, A, B + E);
+            const float E = __builtin_fmaf(1.1920929e-6f, fabsf(B), 3.0398369e-4f * fabsf(A));
+            const float T = __builtin_fmaf(-1024.0f, A, B);
+            Bn = T - E;
+            Bf = T + E;
         };
         float ax, bnx, bfx, ay, bny, bfy, az, bnz, bfz;
         axis(px, q0.w & 0xffu, o.x, inv.x, ax, bnx, bfx);
@@ -307,9 +329,13 @@ struct RayState {
         const half2v hxz[4] = {byte_pair(xz0, 0), byte_pair(xz0, 1), byte_pair(xz1, 0), byte_pair(xz1, 1)};
         // Branch-free child loop.  A hit child ORs (meta >> 5) << (meta & 31)
         // into acc: a leaf's triangle span lands in bits 0-23, an internal
-        // child in slot c sets bit 24 + c.  fmaxf/fminf (v_max3/v_min3) drop
-        // NaN operands, which only widens [tn, tf].
+        // child in slot c sets bit 24 + c, an empty slot (meta 0) nothing.
+        // fmaxf/fminf (v_max3/v_min3) drop NaN operands, which only widens
+        // [tn, tf].  Closest hit: `near1` and `near2` are the least two keys
+        // (tn with the slot in its low bits) of the internal children hit, as
+        // signed integers, so that negative tn sort before all others.
         uint32_t acc = 0;
+        int near1 = 0x7fffffff, near2 = 0x7fffffff;
 #pragma unroll
         for (int c = 0; c < 8; c++) {
             const uint32_t meta = byte_of(q1.z, q1.w, c);
@@ -321,20 +347,45 @@ struct RayState {
             const float tfz = __builtin_fmaf(plane_q(hxz, c), az, bfz);
             const float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin));
             const float tf = fminf(fminf(tfx, tfy), fminf(tfz, t_far));
-            const bool hit = tn <= tf && meta != 0u;
-            acc |= hit ? (meta >> 5) << (meta & 31u) : 0u;
+            const uint32_t w = tn <= tf ? (meta >> 5) << (meta & 31u) : 0u;
+            acc |= w;
+            if (!ANY) {
+                const int key = (int)((__float_as_uint(tn) & ~7u) | (uint32_t)c);
+                const int k = w > 0xffffffu ? key : 0x7fffffff;
+                near2 = med3(near1, k, near2);  // near1 <= near2
+                near1 = min(near1, k);
+            }
         }
         const uint32_t thits = acc & 0xffffffu;
-        // internal hits from slot order (bit c) to visit order (bit c ^ oct)
         uint32_t ihits = acc >> 24;
-        ihits = (oct & 1) ? ((ihits & 0x55u) << 1) | ((ihits >> 1) & 0x55u) : ihits;
-        ihits = (oct & 2) ? ((ihits & 0x33u) << 2) | ((ihits >> 2) & 0x33u) : ihits;
-        ihits = (oct & 4) ? ((ihits & 0x0fu) << 4) | (ihits >> 4) : ihits;
-        // The hit children are visited in octant order, the group kept as one
-        // stack entry.  Choosing the nearest child first visited fewer nodes
-        // (14.1 against 15.3 per ray on the 5.2M-triangle sphere field) but
-        // cost more per node step than it saved (2921 against 2948 Mrays/s).
-        cur = make_uint2(q1.x, (ihits << 24) | imask);
+        // The nearest internal child hit is visited next (any hit: the first
+        // in slot order), the others wait on the stack as one entry.  With
+        // the VALU busy for 0.83 of the time, the kernel is bound by its node
+        // steps: against visits ordered by the ray's octant without bounds,
+        // the 1080p sphere field takes 13.4 node steps per ray (16.4) at 8%
+        // more instructions each, closest hits 12.0 ms of 8 spp (13.1); the
+        // instanced field 11.9 (13.2), 11.2 ms (11.5).  The entry: child
+        // base, hits << 24 | bound << 8 | internal mask, where the bound is
+        // the least tn among them rounded toward zero to 15 bits, zero for
+        // negative ones.  A group whose bound lies beyond the closest hit is
+        // dropped when it is popped.  In a two-level tree a top-level node
+        // that also hit instances pushes its whole group, since the lane
+        // enters those first.
+        if (ihits) {
+            uint32_t bound = 0;
+            if (TWO && top && thits) {
+                if (!ANY) bound = (uint32_t)max(near1, 0);
+            } else {
+                const uint32_t slot = ANY ? (uint32_t)__builtin_ctz(ihits) : (uint32_t)near1 & 7u;
+                next = q1.x + __builtin_popcount(imask & ((1u << slot) - 1u));
+                ihits &= ~(1u << slot);
+                if (!ANY) bound = (uint32_t)max(near2, 0);
+            }
+            if (ihits) {
+                stk.store(sp, make_uint2(q1.x, (ihits << 24) | ((bound >> 8) & 0x7fff00u) | imask));
+                sp++;
+            }
+        }
         if (kTwoSlots && tg.y != 0u) tg2 = make_uint2(q1.y, thits);
         else tg = make_uint2(q1.y, thits);
         return false;
