@@ -328,9 +328,8 @@ void batch_read_image(rm_batch* b, uint32_t job, float* rgba, size_t count) {
     const size_t px = (size_t)ji.width * ji.height;
     RM_REQUIRE(count >= px * 4, "output buffer too small");
     hipStream_t st = b->dev->stream;
-    const float* img = b->renderer->image_buf.as<float>() + (size_t)ji.image_offset * 4;
-    RM_HIP(hipMemcpyAsync(rgba, img, px * 16, hipMemcpyDeviceToHost, st));
-    RM_HIP(hipStreamSynchronize(st));
+    float* img = b->renderer->image_buf.as<float>() + (size_t)ji.image_offset * 4;
+    b->dev->copies->to_host({{rgba, img, px * 16}}, st);
 }
 
 namespace {

@@ -59,6 +59,7 @@ int rm_device_create(int ordinal, rm_device** out) {
     rm_device* d = new rm_device();
     d->ordinal = ordinal;
     try {
+        d->copies = std::make_unique<rm::HostCopies>(ordinal);
         RM_HIP(hipGetDeviceProperties(&d->props, ordinal));
         RM_HIP(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
         d->trace_blocks_per_cu = rm::trace_blocks_per_cu(false);
@@ -76,6 +77,7 @@ int rm_device_create(int ordinal, rm_device** out) {
 
 void rm_device_destroy(rm_device* dev) {
     if (!dev) return;
+    dev->copies.reset();
     if (dev->stream) (void)hipStreamDestroy(dev->stream);
     delete dev;
 }
@@ -182,16 +184,16 @@ int rm_scene_read_envmap(rm_scene* scene, float* pdfs, size_t pdf_count, float* 
     RM_NULL_CHECK(scene);
     RM_GUARD_BEGIN
     RM_REQUIRE(scene->envmap_built, "envmap not built");
-    hipStream_t st = scene->dev->stream;
+    std::vector<rm::CopyPiece> out;
     if (pdfs) {
         RM_REQUIRE(pdf_count * 4 >= scene->d_env_pdfs.bytes, "pdf buffer too small");
-        RM_HIP(hipMemcpyAsync(pdfs, scene->d_env_pdfs.ptr, scene->d_env_pdfs.bytes, hipMemcpyDeviceToHost, st));
+        out.push_back({pdfs, scene->d_env_pdfs.ptr, scene->d_env_pdfs.bytes});
     }
     if (mipmap) {
         RM_REQUIRE(mip_count * 4 >= scene->d_env_mip.bytes, "mipmap buffer too small");
-        RM_HIP(hipMemcpyAsync(mipmap, scene->d_env_mip.ptr, scene->d_env_mip.bytes, hipMemcpyDeviceToHost, st));
+        out.push_back({mipmap, scene->d_env_mip.ptr, scene->d_env_mip.bytes});
     }
-    RM_HIP(hipStreamSynchronize(st));
+    scene->dev->copies->to_host(out, scene->dev->stream);
     RM_GUARD_END
 }
 

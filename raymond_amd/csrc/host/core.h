@@ -16,6 +16,7 @@
 #include "../device/batch.h"
 #include "../device/scene.h"
 #include "../device/camera.h"
+#include "transfer.h"
 
 namespace rm {
 
@@ -120,6 +121,8 @@ struct rm_device {
     // raw ray batches: buffers kept between calls, held by one at a time
     std::mutex raw_mutex;
     rm::RawBuffers raw;
+    // copies between the device and the caller's host memory
+    std::unique_ptr<rm::HostCopies> copies;
 };
 
 struct rm_scene {

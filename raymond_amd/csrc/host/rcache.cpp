@@ -24,9 +24,9 @@ struct InitRng {
 };
 
 // Rows of a raw batch, as the caller has them.
-void stage_rows(DevBuf& buf, const float* rows, size_t floats, hipStream_t s) {
+void stage_rows(rm_cache* c, DevBuf& buf, const float* rows, size_t floats) {
     buf.reserve(floats * 4);
-    RM_HIP(hipMemcpyAsync(buf.ptr, rows, floats * 4, hipMemcpyHostToDevice, s));
+    c->dev->copies->to_device(buf.ptr, rows, floats * 4, c->dev->stream);
 }
 
 void zero_grads(rm_cache* c, hipStream_t s) {
@@ -161,17 +161,18 @@ float cache_step(rm_cache* c, const RcSamples& smp, uint32_t batch, bool read_lo
 
 void cache_read_params(rm_cache* c, float* mlp, size_t mlp_count, float* table, size_t table_count) {
     hipStream_t s = c->dev->stream;
+    std::vector<CopyPiece> out;
     if (mlp) {
         RM_REQUIRE(mlp_count >= (size_t)kRcMlpParams, "mlp buffer too small");
-        RM_HIP(hipMemcpyAsync(mlp, c->w_master.ptr, kRcMlpParams * 4, hipMemcpyDeviceToHost, s));
+        out.push_back({mlp, c->w_master.ptr, kRcMlpParams * 4});
     }
     if (table) {
         RM_REQUIRE(table_count >= c->table_floats, "table buffer too small");
         RM_HIP(launch_rc_table_master(c->t_state.as<float>(), c->t_master.as<float>(), c->t_half.as<uint32_t>(),
                                       c->table_floats, false, s));
-        RM_HIP(hipMemcpyAsync(table, c->t_master.ptr, c->table_floats * 4, hipMemcpyDeviceToHost, s));
+        out.push_back({table, c->t_master.ptr, c->table_floats * 4});
     }
-    RM_HIP(hipStreamSynchronize(s));
+    c->dev->copies->to_host(out, s);
 }
 
 void cache_write_params(rm_cache* c, const float* mlp, size_t mlp_count, const float* table, size_t table_count) {
@@ -182,7 +183,7 @@ void cache_write_params(rm_cache* c, const float* mlp, size_t mlp_count, const f
     }
     if (table) {
         RM_REQUIRE(table_count >= c->table_floats, "table buffer too small");
-        RM_HIP(hipMemcpyAsync(c->t_master.ptr, table, c->table_floats * 4, hipMemcpyHostToDevice, s));
+        c->dev->copies->to_device(c->t_master.ptr, table, c->table_floats * 4, s);
         RM_HIP(launch_rc_table_master(c->t_state.as<float>(), c->t_master.as<float>(), c->t_half.as<uint32_t>(),
                                       c->table_floats, true, s));
     }
@@ -193,7 +194,7 @@ void cache_write_params(rm_cache* c, const float* mlp, size_t mlp_count, const f
 void cache_infer_raw(rm_cache* c, const float* features, uint32_t n, float* out) {
     if (n == 0) return;
     hipStream_t s = c->dev->stream;
-    stage_rows(c->stage_feat, features, (size_t)n * kRcFeatureFloats, s);
+    stage_rows(c, c->stage_feat, features, (size_t)n * kRcFeatureFloats);
     c->stage_out.reserve((size_t)n * 3 * 4);
     RcInferArgs a{};
     a.p = cache_params(c);
@@ -202,14 +203,12 @@ void cache_infer_raw(rm_cache* c, const float* features, uint32_t n, float* out)
     a.out = c->stage_out.as<float>();
     const uint32_t blocks = std::min<uint32_t>((n + 127) / 128, 4096);
     RM_HIP(launch_rc_infer(a, (int)blocks, s));
-    RM_HIP(hipMemcpyAsync(out, c->stage_out.ptr, (size_t)n * 3 * 4, hipMemcpyDeviceToHost, s));
-    RM_HIP(hipStreamSynchronize(s));
+    c->dev->copies->to_host({{out, c->stage_out.ptr, (size_t)n * 3 * 4}}, s);
 }
 
 static RcSamples stage_samples(rm_cache* c, const float* features, const float* targets, uint32_t n) {
-    hipStream_t s = c->dev->stream;
-    stage_rows(c->stage_feat, features, (size_t)n * kRcFeatureFloats, s);
-    stage_rows(c->stage_target, targets, (size_t)n * 3, s);
+    stage_rows(c, c->stage_feat, features, (size_t)n * kRcFeatureFloats);
+    stage_rows(c, c->stage_target, targets, (size_t)n * 3);
     RcSamples smp{};
     smp.feat = c->stage_feat.as<float>();
     smp.target = c->stage_target.as<float>();
@@ -226,11 +225,12 @@ void cache_gradients_raw(rm_cache* c, const float* features, const float* target
     cache_backward(c, smp, n, s);
     if (grad_table) RM_HIP(launch_rc_table_grads(c->t_grad.as<uint32_t>(), c->t_master.as<float>(), c->table_floats, s));
     else RM_HIP(launch_rc_fill(c->t_grad.as<float>(), 0.0f, c->table_floats / 2, s));
-    if (grad_mlp) RM_HIP(hipMemcpyAsync(grad_mlp, c->w_grad.ptr, kRcMlpParams * 4, hipMemcpyDeviceToHost, s));
+    std::vector<CopyPiece> out;
+    if (grad_mlp) out.push_back({grad_mlp, c->w_grad.ptr, kRcMlpParams * 4});
+    if (loss) out.push_back({loss, c->loss.ptr, 4});
+    if (grad_table) out.push_back({grad_table, c->t_master.ptr, c->table_floats * 4});
+    c->dev->copies->to_host(out, s);
     RM_HIP(launch_rc_fill(c->w_grad.as<float>(), 0.0f, kRcMlpParams, s));
-    if (loss) RM_HIP(hipMemcpyAsync(loss, c->loss.ptr, 4, hipMemcpyDeviceToHost, s));
-    if (grad_table)
-        RM_HIP(hipMemcpyAsync(grad_table, c->t_master.ptr, c->table_floats * 4, hipMemcpyDeviceToHost, s));
     RM_HIP(hipStreamSynchronize(s));
 }
 

@@ -772,16 +772,14 @@ void renderer_render(rm_renderer* r, uint32_t samples, rm_render_stats* stats) {
 void renderer_read_image(rm_renderer* r, float* rgba, size_t count) {
     RM_REQUIRE(count >= (size_t)r->width * r->height * 4, "output buffer too small");
     hipStream_t st = r->scene->dev->stream;
-    RM_HIP(hipMemcpyAsync(rgba, r->image_buf.ptr, (size_t)r->width * r->height * 16, hipMemcpyDeviceToHost, st));
-    RM_HIP(hipStreamSynchronize(st));
+    r->scene->dev->copies->to_host({{rgba, r->image_buf.ptr, (size_t)r->width * r->height * 16}}, st);
 }
 
 void renderer_read_image_f64(rm_renderer* r, double* rgba, size_t count) {
     RM_REQUIRE(count >= (size_t)r->width * r->height * 4, "output buffer too small");
     RM_REQUIRE(r->image64_buf.ptr != nullptr, "FP64 accumulation not enabled");
     hipStream_t st = r->scene->dev->stream;
-    RM_HIP(hipMemcpyAsync(rgba, r->image64_buf.ptr, (size_t)r->width * r->height * 32, hipMemcpyDeviceToHost, st));
-    RM_HIP(hipStreamSynchronize(st));
+    r->scene->dev->copies->to_host({{rgba, r->image64_buf.ptr, (size_t)r->width * r->height * 32}}, st);
 }
 
 void renderer_resolve(rm_renderer* r, float* rgba, size_t count) {
@@ -794,8 +792,7 @@ void renderer_resolve(rm_renderer* r, float* rgba, size_t count) {
     const float divisor = (float)(n > 0 ? n : 1);
     RM_HIP(launch_resolve(r->image_buf.as<float>(), r->resolve_buf.as<float>(), r->width * r->height, r->u.exposure,
                           divisor, (int)r->u.tonemapping, st));
-    RM_HIP(hipMemcpyAsync(rgba, r->resolve_buf.ptr, (size_t)r->width * r->height * 16, hipMemcpyDeviceToHost, st));
-    RM_HIP(hipStreamSynchronize(st));
+    r->scene->dev->copies->to_host({{rgba, r->resolve_buf.ptr, (size_t)r->width * r->height * 16}}, st);
 }
 
 }  // namespace rm

@@ -648,7 +648,7 @@ void trace_closest_raw(rm_scene* s, const float* rays, uint32_t n, float* t, uin
     const size_t col = (size_t)n * 4;
     b.in.reserve(col * 8);
     b.out.reserve(col * 5);
-    RM_HIP(hipMemcpyAsync(b.in.ptr, rays, col * 8, hipMemcpyHostToDevice, st));
+    s->dev->copies->to_device(b.in.ptr, rays, col * 8, st);
     // pairs first: 8-byte alignment for any n
     char* o = b.out.as<char>();
     ClosestArgs a{};
@@ -666,11 +666,12 @@ void trace_closest_raw(rm_scene* s, const float* rays, uint32_t n, float* t, uin
     a.spill = s->d_spill.as<uint2>();
     const int blocks = s->dev->props.multiProcessorCount * s->dev->trace_blocks_per_cu;
     RM_HIP(launch_trace_closest(a, blocks, false, st));
-    if (t) RM_HIP(hipMemcpyAsync(t, a.hits.t, col, hipMemcpyDeviceToHost, st));
-    if (inst) RM_HIP(hipMemcpyAsync(inst, a.hits.inst, col, hipMemcpyDeviceToHost, st));
-    if (prim) RM_HIP(hipMemcpyAsync(prim, a.hits.prim, col, hipMemcpyDeviceToHost, st));
-    if (bary) RM_HIP(hipMemcpyAsync(bary, a.bary, 2 * col, hipMemcpyDeviceToHost, st));
-    RM_HIP(hipStreamSynchronize(st));
+    std::vector<CopyPiece> hits;
+    if (t) hits.push_back({t, a.hits.t, col});
+    if (inst) hits.push_back({inst, a.hits.inst, col});
+    if (prim) hits.push_back({prim, a.hits.prim, col});
+    if (bary) hits.push_back({bary, a.bary, 2 * col});
+    s->dev->copies->to_host(hits, st);
 }
 
 void trace_any_raw(rm_scene* s, const float* rays, uint32_t n, uint32_t* occluded) {
@@ -682,7 +683,7 @@ void trace_any_raw(rm_scene* s, const float* rays, uint32_t n, uint32_t* occlude
     const size_t col = (size_t)n * 4;
     b.in.reserve(col * 8);
     b.out.reserve(col);
-    RM_HIP(hipMemcpyAsync(b.in.ptr, rays, col * 8, hipMemcpyHostToDevice, st));
+    s->dev->copies->to_device(b.in.ptr, rays, col * 8, st);
     AnyArgs a{};
     a.nodes = s->d_nodes.as<Bvh8Node>();
     a.tris = s->d_tris.as<BvhTri>();
@@ -695,8 +696,7 @@ void trace_any_raw(rm_scene* s, const float* rays, uint32_t n, uint32_t* occlude
     a.spill = s->d_spill.as<uint2>();
     const int blocks = s->dev->props.multiProcessorCount * s->dev->any_blocks_per_cu;
     RM_HIP(launch_trace_any(a, blocks, false, st));
-    RM_HIP(hipMemcpyAsync(occluded, b.out.ptr, col, hipMemcpyDeviceToHost, st));
-    RM_HIP(hipStreamSynchronize(st));
+    s->dev->copies->to_host({{occluded, b.out.ptr, col}}, st);
 }
 
 }  // namespace rm

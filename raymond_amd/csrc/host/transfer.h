@@ -1,0 +1,83 @@
+// Copies between the device and pageable host memory of the caller.
+//
+// A plain hipMemcpyAsync into memory that the caller has just allocated is
+// bound by one thread's page faults and memcpy: 33 MB take 2.4 ms, four times
+// the DMA's 0.6 ms.  HostCopies moves such copies in blocks through a ring of
+// pinned slots, where the DMA of one block overlaps the memcpy of others by a
+// few worker threads.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <condition_variable>
+#include <cstdint>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace rm {
+
+struct CopyPiece {
+    void* host;
+    void* device;
+    size_t bytes;
+};
+
+class HostCopies {
+public:
+    explicit HostCopies(int ordinal) : ordinal_(ordinal) {}
+    HostCopies(const HostCopies&) = delete;
+    HostCopies& operator=(const HostCopies&) = delete;
+    ~HostCopies();
+
+    // Copies in the stream's order; returns when the host has the data.
+    void to_host(const std::vector<CopyPiece>& pieces, hipStream_t st);
+    // Copies in the stream's order; returns when the host memory may change.
+    void to_device(void* device, const void* host, size_t bytes, hipStream_t st);
+
+private:
+    // a DMA's worth of the copy, one slot: one transfer per piece in it
+    struct Part {
+        size_t slot_offset;
+        char* device;
+        size_t bytes;
+    };
+    struct Block {
+        size_t parts_end, chunks_end;  // in parts_, chunks_
+    };
+    // one worker's memcpy
+    struct Chunk {
+        size_t block, slot_offset;
+        char* host;
+        size_t bytes;
+    };
+    bool staged(const std::vector<CopyPiece>& pieces) const;
+    bool prepare();
+    void cut(const std::vector<CopyPiece>& pieces);
+    void begin(const std::vector<CopyPiece>& pieces, bool to_host);
+    void transfer(size_t block, hipStream_t st);
+    void release_block(size_t block);
+    void drain();
+    void wait_finished(size_t block);
+    bool is_finished(size_t block);
+    void wait_slot(size_t slot);
+    void work();
+
+    const int ordinal_;
+    std::mutex in_use_;  // one staged copy at a time
+    bool prepared_ = false, usable_ = false;
+    char* slots_ = nullptr;
+    std::vector<hipEvent_t> events_;
+    std::vector<uint8_t> pending_;  // the slot's DMA has been enqueued and not waited for
+    std::vector<std::thread> workers_;
+
+    // the copy in hand, shared with the workers
+    std::mutex mutex_;
+    std::condition_variable wake_, finished_cv_;
+    std::vector<Part> parts_;
+    std::vector<Chunk> chunks_;
+    std::vector<Block> blocks_;
+    std::vector<size_t> unfinished_;  // per block: chunks not yet copied
+    size_t released_ = 0, claimed_ = 0, finished_count_ = 0;
+    bool to_host_ = false, stop_ = false;
+};
+
+}  // namespace rm
