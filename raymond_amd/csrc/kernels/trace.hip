@@ -92,15 +92,13 @@ struct StackRef {
     }
 };
 
-// Postponed leaf sets a lane may hold while it takes nodes (1 or 2), and the
-// share of a wave's active lanes held up by their triangles (1/kHeldShare)
-// that starts a triangle phase.  On the 5.2M-triangle sphere field
-// (Mrays/s, against 2944-2976 for one slot at a quarter): two slots at 1/4
-// 3035, 1/5 3049, 1/6 3037-3071, 1/8 3051, 1/12 3018, 1/16 2996; at 1/3
-// 2935 and 1/2 2773.  Two slots visit more nodes per ray (16.1 against
-// 15.3: closer hits arrive later) but keep more lanes busy.  Three slots
-// measured 2875 (at 1/6 and 1/8): 16.9 nodes per ray, and the closest-hit
-// kernel's 97 VGPRs fit 4 waves per SIMD.
+// Postponed leaf sets a lane of a flat tree may hold while it takes nodes (1
+// or 2), and the share of a wave's active lanes held up by their triangles
+// (1/kHeldShare) that starts a triangle phase.  On the 5.2M-triangle sphere
+// field, 8 spp in ms: two slots at 1/4 24.98, 1/5 24.83, 1/6 24.74, 1/8 24.91;
+// one slot at 1/4 25.06.  Two slots visit more nodes per ray (13.4 against
+// 12.7: closer hits arrive later) but keep more lanes busy.  Three slots
+// measured less: the closest-hit kernel then fits 4 waves per SIMD.
 #ifndef RM_LEAF_SLOTS
 #define RM_LEAF_SLOTS 2
 #endif
@@ -109,15 +107,29 @@ constexpr int kLeafSlots = RM_LEAF_SLOTS;
 #define RM_HELD_SHARE 6
 #endif
 constexpr int kHeldShare = RM_HELD_SHARE;
+// In a two-level tree a lane holds one leaf set: its lanes are held up by
+// instances to enter as well, and 0.3 fewer nodes and 0.2 fewer triangles per
+// ray weigh more than the lanes that a second set would keep busy.  1080p
+// instanced field, 8 spp in ms: two slots at 1/6 17.70 (1/4 17.66, 1/8 17.82),
+// one slot at 1/6 17.49, 1/5 17.43, 1/4 17.24, 1/3 17.11, 1/2 17.53.
+#ifndef RM_HELD_SHARE_2L
+#define RM_HELD_SHARE_2L 3
+#endif
+constexpr int kHeldShare2l = RM_HELD_SHARE_2L;
 // The any-hit kernel, whose rays may end at their first hit, starts its
-// triangle phases sooner: at 1/3 with 3 triangles per phase, its time on
-// the sphere field measured 0.341-0.343 ms per spp against 0.353-0.354 at
-// the closest-hit kernel's 1/6 and 2 (1/4 and 3: 0.342-0.344; 1/4 and 4:
-// 0.342-0.344, slower on the instanced field; 1/10 and 2: 0.363).
+// triangle phases sooner.  Flat tree: at 1/4 with 2 triangles per phase the
+// sphere field's shadow rays take 6.19 ms of 8 spp (1/3 and 3: 6.44, 1/5 and
+// 2: 6.17, 1/6 and 2: 6.20, 1/4 and 4: 6.20, 1/4 and 1: 6.47, 1/2 and 3:
+// 6.89).  Two-level tree: at 1/3 with 3 per phase the instanced field's take
+// 4.21 (1/4 and 2: 4.41, 1/2 and 3: 4.48).
 #ifndef RM_HELD_SHARE_ANY
-#define RM_HELD_SHARE_ANY 3
+#define RM_HELD_SHARE_ANY 4
 #endif
 constexpr int kHeldShareAny = RM_HELD_SHARE_ANY;
+#ifndef RM_HELD_SHARE_ANY_2L
+#define RM_HELD_SHARE_ANY_2L 3
+#endif
+constexpr int kHeldShareAny2l = RM_HELD_SHARE_ANY_2L;
 
 // Traversal state of one lane's ray.  It persists across steps, so a lane
 // whose ray has finished takes a new one while the rest of the wave goes on.
@@ -132,13 +144,12 @@ struct RayState {
     bool found;
     uint32_t next;  // node to visit, or kNoNode
     uint2 tg;   // postponed leaf triangles: base, mask (top level of a two-level tree: instances)
-    uint2 tg2;  // a second postponed leaf set (kLeafSlots == 2)
+    uint2 tg2;  // a second postponed leaf set (flat trees, kLeafSlots == 2)
     int sp;
     uint32_t n_nodes, n_tris;
     // two-level trees: the instance entered, in the top level
     uint32_t inst;
     bool top;
-    int marker_sp;  // stack index of the instance's marker entry (-1 in the top level)
 
     __device__ void set_ray(vec3 org, vec3 d) {
         o = org;
@@ -150,7 +161,6 @@ struct RayState {
         set_ray(org, d);
         inst = 0;
         top = true;
-        marker_sp = -1;
         next = root;
         sp = 0;
         tmin = t0;
@@ -186,7 +196,6 @@ struct RayState {
         const uint4* ip = reinterpret_cast<const uint4*>(insts + tg.x + (uint32_t)b);
         const uint4 r0 = ip[0], r1 = ip[1], r2 = ip[2], r3 = ip[3];
         stk.store(sp, make_uint2(tg.x, kMarker2l | tg.y));
-        marker_sp = sp;
         sp++;
         TlasInstance ti;
         const uint4 rows[3] = {r0, r1, r2};
@@ -219,16 +228,17 @@ struct RayState {
         // with one is held like a lane with triangles and enters the next
         // instance in the same phase as the others test triangles, so the
         // entry code runs for many lanes at once rather than in most steps
-        // for a few.  A lane tests its pending triangles before it pops its
-        // instance's marker: they belong to the instance's ray.
-        constexpr bool kTwoSlots = kLeafSlots > 1;
+        // for a few.  With its one slot, a lane tests its pending triangles
+        // before it pops its instance's marker: they belong to the instance's
+        // ray.
+        constexpr bool kTwoSlots = !TWO && kLeafSlots > 1;
+        constexpr int kShare = ANY ? (TWO ? kHeldShareAny2l : kHeldShareAny) : (TWO ? kHeldShare2l : kHeldShare);
         const bool to_enter = TWO && top && tg.y != 0u;
         const bool has_tris = !to_enter && tg.y != 0u;
         const bool node_work = next != kNoNode || sp > 0;
-        bool can_node = !to_enter && node_work && (kTwoSlots ? tg2.y == 0u : !has_tris);
-        if (TWO && kTwoSlots && has_tris && next == kNoNode && sp - 1 == marker_sp) can_node = false;
+        const bool can_node = !to_enter && node_work && (kTwoSlots ? tg2.y == 0u : !has_tris);
         const unsigned long long held = __ballot((has_tris || to_enter) && !can_node);
-        if (__popcll(held) * (ANY ? kHeldShareAny : kHeldShare) >= __popcll(__ballot(true)) ||
+        if (__popcll(held) * kShare >= __popcll(__ballot(true)) ||
             __ballot(can_node) == 0ull) {
             if (to_enter) {
                 enter(insts, stk);
@@ -258,11 +268,6 @@ struct RayState {
                 if (!ANY && !TWO && beyond(e)) return false;
             } while (!ANY && TWO && beyond(e));
             if (TWO && (e.y & kMarker2l)) {
-                // pending triangles belong to the instance's ray
-                if (kTwoSlots && has_tris) {
-                    sp++;
-                    return false;
-                }
                 // back in the world: the set's other instances, then the
                 // top-level groups below the marker (entering the next
                 // instance maps the ray again, so the world ray is needed only
@@ -270,8 +275,7 @@ struct RayState {
                 tg = make_uint2(e.x, e.y & ~kMarker2l);
                 if (tg.y == 0u) set_ray(stk.world_o(), stk.world_d());
                 top = true;
-                marker_sp = -1;
-                return false;
+                        return false;
             }
             const uint32_t hits = e.y >> 24;
             const uint32_t rest = hits & (hits - 1u);
@@ -403,14 +407,18 @@ struct RayState {
 #define RM_TRIS_PER_PHASE 2
 #endif
     static constexpr int kTrisPerPhase = RM_TRIS_PER_PHASE;
-// (any hit: 1 per phase 0.380 ms per spp against 0.354 for 2, 3 0.349-0.350)
+// (any hit: measured with the shares above)
 #ifndef RM_TRIS_PER_PHASE_ANY
-#define RM_TRIS_PER_PHASE_ANY 3
+#define RM_TRIS_PER_PHASE_ANY 2
 #endif
     static constexpr int kTrisPerPhaseAny = RM_TRIS_PER_PHASE_ANY;
+#ifndef RM_TRIS_PER_PHASE_ANY_2L
+#define RM_TRIS_PER_PHASE_ANY_2L 3
+#endif
+    static constexpr int kTrisPerPhaseAny2l = RM_TRIS_PER_PHASE_ANY_2L;
     template <bool ANY, bool STATS, bool TWO>
     __device__ bool test_tris(const BvhTri* __restrict__ tris) {
-        for (int k = 0; k < (ANY ? kTrisPerPhaseAny : kTrisPerPhase) && tg.y; k++) {
+        for (int k = 0; k < (ANY ? (TWO ? kTrisPerPhaseAny2l : kTrisPerPhaseAny) : kTrisPerPhase) && tg.y; k++) {
             const int b = __builtin_ctz(tg.y);
             tg.y &= tg.y - 1u;
             const uint4* tp = reinterpret_cast<const uint4*>(tris + tg.x + b);
