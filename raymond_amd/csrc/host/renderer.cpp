@@ -436,9 +436,9 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
     bool drain = total <= r->capacity;
     uint32_t last = drain ? r->max_depth : ~0u;
 
-    // One iteration: regenerate, closest hit (with the previous iteration's
-    // shadow rays), material sort, shade.  Directly launched, `it` is the
-    // iteration; inside a captured chunk it is the offset from the device
+    // One iteration: regenerate and closest hit (with the previous iteration's
+    // shadow rays), then material sort and shade.  Directly launched, `it` is
+    // the iteration; inside a captured chunk it is the offset from the device
     // counter iter_base (chunks start at even iterations, so the queue parity
     // is the offset's).
     const uint32_t* iter_dev = nullptr;
@@ -446,9 +446,8 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
         aa.shadows.slot = cache_train ? r->shadow_slot_buf.as<uint32_t>() : nullptr;
         aa.slot_radiance = cache_train ? r->cv.slot_radiance : nullptr;
     }
-    auto enqueue = [&](uint32_t it) {
+    auto enqueue_trace = [&](uint32_t it) {
         PathQueue& cur = r->q[it & 1];
-        PathQueue& next = r->q[(it + 1) & 1];
         ca.drain = drain && !iter_dev && it > 0;
         if (!ca.drain) {
             ga.iter = it;
@@ -467,6 +466,17 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
             RM_HIP(launch_trace_closest(ca, tblocks, tstats, st));
             tm.end(e, tm.closest);
         }
+    };
+    auto enqueue_any = [&](uint32_t it) {
+        aa.iter = it;
+        aa.iter_dev = iter_dev;
+        hipEvent_t ea = tm.begin();
+        RM_HIP(launch_trace_any(aa, ablocks, tstats, st));
+        tm.end(ea, tm.any);
+    };
+    auto enqueue_shade = [&](uint32_t it) {
+        PathQueue& cur = r->q[it & 1];
+        PathQueue& next = r->q[(it + 1) & 1];
         if (sorting) {
             so.iter = it;
             so.iter_dev = iter_dev;
@@ -499,14 +509,18 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
         hipEvent_t es = tm.begin();
         RM_HIP(hipModuleLaunchKernel(shade_fn, sblocks, 1, 1, 256, 1, 1, 0, st, args, nullptr));
         tm.end(es, tm.shade);
-        if (!merged) {
-            aa.iter = it;
-            aa.iter_dev = iter_dev;
-            hipEvent_t ea = tm.begin();
-            RM_HIP(launch_trace_any(aa, ablocks, tstats, st));
-            tm.end(ea, tm.any);
-        }
+        if (!merged) enqueue_any(it);
     };
+    // What a chunk holds of iteration `it`: its shading and the trace of the
+    // next one, or after the loop's last iteration its shadow rays alone.  A
+    // chunk thus ends with every shadow ray of its iterations traced, and the
+    // done counts copied there are of finished paths.
+    auto enqueue = [&](uint32_t it, bool end) {
+        enqueue_shade(it);
+        if (!end) enqueue_trace(it + 1);
+        else if (merged) enqueue_any(it);
+    };
+    enqueue_trace(0);
 
     // Captured bounce loop: a chunk of kIterChunk iterations and the advance
     // of iter_base, recorded once per stream and replayed until it drains.
@@ -517,7 +531,7 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
         hipGraph_t g = nullptr;
         RM_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         try {
-            for (uint32_t c = 0; c < kIterChunk; c++) enqueue(c);
+            for (uint32_t c = 0; c < kIterChunk; c++) enqueue(c, false);
             RM_HIP(launch_advance_iter(cnt, kIterChunk, st));
         } catch (...) {
             (void)hipStreamEndCapture(st, &g);
@@ -550,7 +564,7 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
             iter += kIterChunk;
         } else {
             const uint32_t n = std::min(drain && iter > 0 ? kTailChunk : kIterChunk, last - iter);
-            for (uint32_t c = 0; c < n; c++, iter++) enqueue(iter);
+            for (uint32_t c = 0; c < n; c++, iter++) enqueue(iter, iter + 1 == last);
         }
         chunk_end[slot] = iter;
         if (iter >= last && !br) return;  // nothing left to check
@@ -562,18 +576,12 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
     enqueue_chunk(0);
     for (;;) {
         if (iter >= last) {
-            // the loop ends with what is enqueued; its last shadow rays have
-            // no next iteration to go with
+            // the loop ends with what is enqueued
             if (br) {
                 RM_HIP(hipEventSynchronize(lp.ready[slot]));
                 batch_poll_counts(br, lp.done(slot));
             }
             chunk_end[slot] = iter;
-            if (merged) {
-                aa.iter = iter - 1;
-                aa.iter_dev = nullptr;
-                RM_HIP(launch_trace_any(aa, ablocks, false, st));
-            }
             break;
         }
         enqueue_chunk(slot ^ 1);  // runs while the host reads the previous chunk's counters
@@ -588,8 +596,8 @@ static void render_stream(rm_renderer* r, uint32_t samples, rm_render_stats* sta
         }
         slot ^= 1;
     }
-    // a chunk after the last one holds no work but the last shadow rays: the
-    // stream's statistics and stage timers end with the chunk that drained it
+    // a chunk after the last one holds no work: the stream's statistics and
+    // stage timers end with the chunk that drained it
     iter = chunk_end[slot];
     for (auto* v : {&tm.closest, &tm.sort, &tm.shade, &tm.any})
         if (v->size() > iter) v->resize(iter);

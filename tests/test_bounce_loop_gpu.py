@@ -37,3 +37,33 @@ def test_depths_and_launches(cornell, depth, spl, samples):
             assert st.total_rays == res.total_rays
             assert st.shadow_total == sum(res.shadow_rays[d] for d in range(32))
             parity.assert_radiance_close(r.image(), ref)
+
+
+def test_job_times_include_the_last_shadow_rays(device):
+    """A job is complete when its shadow rays are: its time is not read before
+    they are traced.  In a closed room of albedo 2e-6 the weight of a path
+    underflows to zero (2e-6^8 = 2.6e-46) in the shading of iteration 7, the
+    last of the first chunk that the host checks: every path ends there, a
+    third of them with a shadow ray, whose launch takes 0.4 ms.  The launches
+    after it are empty."""
+    desc = scenes.tessellated_cornell_box(256, 256, 200000)
+    desc.envmap_resolution = 64
+    desc.surface_materials = [scenes.diffuse_material("dark", (2e-6, 2e-6, 2e-6))] * 4 + [
+        scenes.emission_material("light", (1.0, 1.0, 1.0), 1e6)]
+    lo, hi = -3.0, 4.0
+    c = [(x, y, z) for x in (lo, hi) for y in (lo, hi) for z in (lo, hi)]
+    desc.add_entity(desc.add_shape(scenes.merge(
+        [scenes.quad(*(c[k] for k in q), 0) for q in ((0, 2, 6, 4), (1, 5, 7, 3), (0, 4, 5, 1), (2, 3, 7, 6),
+                                                      (0, 1, 3, 2), (4, 6, 7, 5))])))
+    scene = scenes.build_device_scene(device, desc)
+    b = api.Batch(device, [(scene, 256, 256, 60, 12, 1)])
+    st = b.render(rr_depth=64, timing=1)
+    assert st.iterations >= 8 and st.ms_trace_any > 1.0
+    launch = st.ms_trace_any / 8
+    gaps = []
+    for _ in range(5):
+        st = b.render(rr_depth=64)
+        assert b.job_times()[0] == st.makespan_ms
+        gaps.append(st.ms_total - st.makespan_ms)
+    print("from the job's time to the end %.3f ms, shadow rays of an iteration %.3f ms" % (min(gaps), launch))
+    assert min(gaps) < 0.5 * launch
