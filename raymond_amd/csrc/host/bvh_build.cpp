@@ -259,7 +259,8 @@ struct Collapse {
             const double internal = area * kCostNode + dist[8];
             const double leaf = count[n] <= max_leaf ? area * kCostTri * count[n] : INFINITY;
             c[0] = (float)std::min(internal, leaf);
-            h[0] = leaf <= internal ? 0 : 1;
+            // both are infinite where the area overflows a float
+            h[0] = count[n] <= max_leaf && leaf <= internal ? 0 : 1;
             for (int i = 2; i <= 8; i++) {
                 if (dist[i] < (double)c[i - 2]) {
                     c[i - 1] = (float)dist[i];

@@ -771,7 +771,7 @@ __device__ inline void collapse_node(double area, uint32_t count, uint32_t max_l
     const double internal = area * kCostNode + dist[8];
     const double leaf = count <= max_leaf ? area * kCostTri * count : __builtin_huge_val();
     c[0] = (float)fmin(internal, leaf);
-    uint64_t h = leaf <= internal ? 0 : 1;
+    uint64_t h = count <= max_leaf && leaf <= internal ? 0 : 1;
 #pragma unroll
     for (int i = 2; i <= 8; i++) {
         if (dist[i] < (double)c[i - 2]) {

@@ -43,6 +43,14 @@ def repeated(rng, n):
     return np.repeat(soup(rng, 7), (n + 6) // 7, axis=0)[:n]
 
 
+def huge(rng, n):
+    """A soup and a few triangles so far away that the areas of the nodes
+    above them overflow a float."""
+    t = soup(rng, n)
+    t[::n // 6] *= 1e28
+    return t
+
+
 def slivers(rng, n):
     """A third of the triangles without area."""
     t = soup(rng, n)
@@ -92,7 +100,7 @@ def rays_at(tris, rng, n):
 
 CASES = [(soup, 511, 1), (soup, 512, 1), (soup, 1024, 1), (soup, 1025, 3), (soup, 4096, 1), (soup, 4097, 2), (soup, 8193, 1), (soup, 50021, 5),
          (coincident, 1031, 1), (coincident, 4500, 1), (clusters, 20011, 1), (flat, 4160, 2), (repeated, 4300, 1),
-         (slivers, 3001, 1)]
+         (slivers, 3001, 1), (huge, 700, 1), (huge, 4500, 2)]
 
 
 @pytest.mark.parametrize("make,n,instances", CASES, ids=lambda x: getattr(x, "__name__", str(x)))

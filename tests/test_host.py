@@ -111,6 +111,16 @@ def test_bvh8_builder_is_conservative(kind):
     assert nodes >= 1 and depth >= 1
 
 
+@pytest.mark.parametrize("scale", [3e19, 1e20, 1e30, 1e37])
+def test_bvh8_builder_where_areas_overflow(scale):
+    """Node areas beyond the largest float around an ordinary soup: collapse
+    costs are infinite there, which must not make a leaf of them."""
+    tris = random_soup(700, 7)
+    tris[::100] *= scale / 10
+    nodes, depth = api.bvh8_check(tris)
+    assert nodes > 1 and depth < 60
+
+
 def test_bvh8_builder_cornell_and_spheres():
     for desc in (scenes.cornell_box(8, 8), scenes.sphere_field(8, 8, grid=3, level=4)):
         verts, _, _, faces, _, inst = desc.arrays()
