@@ -296,6 +296,7 @@ static bool build_on_device(rm_scene* s, const std::vector<BvhSource>& sources, 
     if (status == kBvhUnsupported) return false;
     RM_REQUIRE(status != kBvhTooDeep, "BVH build failed: BVH8 too deep for the traversal stack");
     RM_REQUIRE(status != kBvhQuantisation, "BVH build failed: BVH8 quantisation failed");
+    scratch.release();  // larger than the nodes, which may fit only now
     nodes.alloc((size_t)num_nodes * sizeof(Bvh8Node));
     RM_HIP(hipMemcpyAsync(nodes.ptr, all_nodes.ptr, nodes.bytes, hipMemcpyDeviceToDevice, st));
     RM_HIP(hipStreamSynchronize(st));
@@ -330,6 +331,10 @@ void scene_build_accel(rm_scene* s, int threads) {
         std::string err;
         Bvh8Build b = build_bvh8(world_triangles(s), threads, &err);
         RM_REQUIRE(err.empty(), "BVH build failed: " + err);
+        // the new tree may not fit beside the old one
+        s->accel_built = false;
+        s->d_nodes.release();
+        s->d_tris.release();
         nodes.upload(b.nodes.data(), b.nodes.size() * sizeof(Bvh8Node), st);
         tris.upload(b.tris.data(), b.tris.size() * sizeof(BvhTri), st);
         RM_HIP(hipStreamSynchronize(st));

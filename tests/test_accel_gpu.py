@@ -4,6 +4,11 @@ any hits through it equal the oracle's exhaustive search bit for bit, at the
 sizes where the builder's phases meet (64 and 1024 triangles per range, 4096
 per workgroup, the smallest device build) and for geometry that leaves nothing to split on.
 Hits do not depend on the tree, so equality needs no tolerance."""
+import json
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -144,3 +149,20 @@ def test_geometry_that_is_not_finite_takes_the_host_builder(device):
     d = description(tris, 1)
     with pytest.raises(api.RmError, match="quantisation failed"):
         api.Scene(device, d).build_accel()
+
+
+def test_builds_with_little_device_memory(device, tmp_path):
+    """Where the device builder's arrays do not fit, or the new tree does not
+    fit beside the old one, a build still succeeds; one that cannot succeed is
+    an error and leaves the scene without a tree."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    shim = str(tmp_path / "malloc_budget.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-o", shim,
+                    os.path.join(here, "native", "malloc_budget.cpp"), "-ldl"], check=True)
+    p = subprocess.run([sys.executable, "-m", "tests.memory_check", shim], cwd=os.path.dirname(here),
+                       capture_output=True, text=True, timeout=90)
+    assert p.returncode == 0, p.stdout + p.stderr
+    out = json.loads(p.stdout.strip().splitlines()[-1])
+    assert "out of memory" in out.pop("no room")
+    assert "not built" in out.pop("trace")
+    assert len(out) == 4 and all(v is True for v in out.values()), out
