@@ -518,6 +518,7 @@ void scene_build_accel_two_level(rm_scene* s, int threads) {
         return true;
     };
     const TwoLevelBuild b = build_two_level(s->vertices, s->indices, s->inst_desc, threads, shape_tree);
+    s->accel_built = false;  // until the new arrays are there: uploading frees the old ones first
     s->d_nodes.upload(b.nodes.data(), b.nodes.size() * sizeof(Bvh8Node), st);
     s->d_tris.upload(b.tris.data(), b.tris.size() * sizeof(BvhTri), st);
     s->d_tlas.upload(b.recs.data(), b.recs.size() * sizeof(TlasInstance), st);

@@ -50,17 +50,20 @@ def main(path):
     rebuild("no room for the scratch arrays", tree + (1 << 20))
     rebuild("room for the device build alone", sum(sizes[:4]))
     rebuild("no room beside the old tree", tree // 2)
-    other = api.Scene(dev, d)
-    shim.budget_room(tree // 2)
-    for name, call in (("no room", other.build_accel), ("trace", lambda: other.trace_closest(rays))):
-        try:
-            call()
-            out[name] = True
-        except api.RmError as e:
-            out[name] = str(e)
-    shim.budget_off()
-    other.build_accel()
-    out["room again"] = all(np.array_equal(a, b) for a, b in zip(hits, other.trace_closest(rays)))
+    first, again = api.Scene(dev, d), api.Scene(dev, d)
+    again.build_accel(two_level=True)
+    for form, other, room in (("flat", first, tree // 2), ("two-level", again, -tree)):  # less than was in use
+        shim.budget_room(room % (1 << 64))
+        for name, call in (("no room", lambda: other.build_accel(two_level=form != "flat")),
+                           ("trace", lambda: other.trace_closest(rays))):
+            try:
+                call()
+                out[form + ", " + name] = True
+            except api.RmError as e:
+                out[form + ", " + name] = str(e)
+        shim.budget_off()
+        other.build_accel()
+        out[form + ", room again"] = all(np.array_equal(a, b) for a, b in zip(hits, other.trace_closest(rays)))
     print(json.dumps(out), flush=True)
 
 

@@ -163,6 +163,7 @@ def test_builds_with_little_device_memory(device, tmp_path):
                        capture_output=True, text=True, timeout=90)
     assert p.returncode == 0, p.stdout + p.stderr
     out = json.loads(p.stdout.strip().splitlines()[-1])
-    assert "out of memory" in out.pop("no room")
-    assert "not built" in out.pop("trace")
-    assert len(out) == 4 and all(v is True for v in out.values()), out
+    for form in ("flat", "two-level"):
+        assert "out of memory" in out.pop(form + ", no room")
+        assert "not built" in out.pop(form + ", trace")
+    assert len(out) == 5 and all(v is True for v in out.values()), out
