@@ -44,6 +44,12 @@ void rmh_free(void* p);
  * (A test hook for the builder behind rm_scene_build_accel.) */
 int rmh_bvh8_check(const float* tris, uint32_t n, int threads, uint32_t* out_nodes, uint32_t* out_depth, char* err,
                    size_t err_cap);
+/* Reads a scene's flat acceleration structure back from the device and
+ * verifies it as rmh_bvh8_check does, its leaf triangles against the scene's;
+ * out_different receives the nodes that differ in any byte from the host
+ * builder's tree over the same triangles, or whose leaves hold others.
+ * Returns 0, or -1 and a message.  (A test hook for rm_scene_build_accel.) */
+int rmh_scene_check_accel(rm_scene* scene, int threads, uint32_t* out_different, char* err, size_t err_cap);
 /* Builds the two-level form of rm_scene_build_accel_two_level on the host
  * from scene arrays (vertices 3 floats each, faces 3 indices relative to the
  * instance's vertex_offset, instance descriptions) and traces n rays (8

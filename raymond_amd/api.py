@@ -238,6 +238,7 @@ EXPORTS = {
     "rmh_jit_precompile": (C.c_int, [C.c_char_p, C.c_size_t, C.c_char_p, C.POINTER(C.c_int), C.c_char_p, C.c_size_t]),
     "rmh_bvh8_check": (C.c_int, [C.c_void_p, C.c_uint32, C.c_int, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32),
                                  C.c_char_p, C.c_size_t]),
+    "rmh_scene_check_accel": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_uint32), C.c_char_p, C.c_size_t]),
     "rmh_two_level_trace": (C.c_int, [C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32,
                                       C.c_void_p, C.c_uint32, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p,
                                       C.c_void_p, C.POINTER(C.c_uint64), C.c_char_p, C.c_size_t]),
@@ -457,6 +458,15 @@ class Scene:
             _check(LIB.rm_scene_build_accel_two_level(self.handle, threads))
         else:
             _check(LIB.rm_scene_build_accel(self.handle, threads))
+
+    def check_accel(self, threads=0):
+        """Verifies the flat tree on the device; returns how many of its nodes
+        differ from the host builder's (rmh_scene_check_accel)."""
+        different = C.c_uint32(0)
+        err = C.create_string_buffer(256)
+        if LIB.rmh_scene_check_accel(self.handle, threads, C.byref(different), err, 256) != 0:
+            raise RmError(err.value.decode())
+        return int(different.value)
 
     def compile_materials(self, source, options=""):
         log = C.create_string_buffer(1 << 16)

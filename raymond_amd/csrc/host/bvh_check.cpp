@@ -1,6 +1,8 @@
-// Host-only structural check of the BVH8 builder: every triangle appears once
-// in the leaves and every decoded (quantised) child box contains the exact
-// bounds of its subtree.  Exposed through include/rm_host.h for tests.
+// Structural check of BVH8 trees, built on the host or read back from the
+// device: every triangle appears once in the leaves and every decoded
+// (quantised) child box contains the exact bounds of its subtree.  Exposed
+// through include/rm_host.h for tests.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -95,8 +97,70 @@ struct Checker {
     }
 };
 
+// The (instance, primitive) pairs of a leaf slot, in order.
+std::vector<std::pair<uint32_t, uint32_t>> leaf_ids(const Bvh8Build& b, const Bvh8Node& n, int slot) {
+    std::vector<std::pair<uint32_t, uint32_t>> ids;
+    const uint32_t first = n.tri_base + (n.meta[slot] & 31u);
+    for (uint32_t bits = n.meta[slot] >> 5, t = first; bits; bits >>= 1, t++) ids.push_back({b.tris[t].inst, b.tris[t].prim});
+    std::sort(ids.begin(), ids.end());
+    return ids;
+}
+
 }  // namespace
 }  // namespace rm
+
+extern "C" int rmh_scene_check_accel(rm_scene* s, int threads, uint32_t* out_different, char* err, size_t err_cap) {
+    try {
+        RM_REQUIRE(s && s->accel_built && !s->two_level, "a scene with a flat acceleration structure is needed");
+        rm::Bvh8Build b;
+        b.nodes.resize(s->stats.bvh_nodes);
+        b.tris.resize(s->stats.triangles);
+        RM_HIP(hipMemcpy(b.nodes.data(), s->d_nodes.ptr, b.nodes.size() * sizeof(rm::Bvh8Node), hipMemcpyDeviceToHost));
+        if (!b.tris.empty())
+            RM_HIP(hipMemcpy(b.tris.data(), s->d_tris.ptr, b.tris.size() * sizeof(rm::BvhTri), hipMemcpyDeviceToHost));
+        rm::Checker c{b, std::vector<int>(b.tris.size(), 0), "", 0};
+        if (!b.tris.empty()) c.node(0, 1);
+        RM_REQUIRE(c.err.empty(), c.err);
+        for (int n : c.seen) RM_REQUIRE(n == 1, "leaf triangle referenced " + std::to_string(n) + " times");
+        // the triangles are the scene's, each once
+        const std::vector<rm::BuildTri> in = rm::world_triangles(s);
+        RM_REQUIRE(in.size() == b.tris.size(), "leaf triangle count differs from the scene's");
+        std::vector<const rm::BvhTri*> leaf;
+        for (const rm::BvhTri& t : b.tris) leaf.push_back(&t);
+        std::sort(leaf.begin(), leaf.end(), [](const rm::BvhTri* x, const rm::BvhTri* y) {
+            return x->inst != y->inst ? x->inst < y->inst : x->prim < y->prim;
+        });
+        for (size_t i = 0; i < in.size(); i++) {
+            const rm::BvhTri& t = *leaf[i];
+            const float v[9] = {in[i].v0.x, in[i].v0.y, in[i].v0.z, in[i].v1.x, in[i].v1.y,
+                                in[i].v1.z, in[i].v2.x, in[i].v2.y, in[i].v2.z};
+            const float w[9] = {t.v0x, t.v0y, t.v0z, t.v1x, t.v1y, t.v1z, t.v2x, t.v2y, t.v2z};
+            RM_REQUIRE(t.inst == in[i].inst && t.prim == in[i].prim && std::memcmp(v, w, sizeof(v)) == 0,
+                       "leaf triangle " + std::to_string(i) + " differs from the scene's");
+        }
+        // against the host builder's tree, node by node
+        std::string e;
+        const rm::Bvh8Build h = rm::build_bvh8(in, threads, &e);
+        RM_REQUIRE(e.empty(), e);
+        uint32_t different = 0;
+        for (size_t i = 0; i < std::max(b.nodes.size(), h.nodes.size()); i++) {
+            bool same = i < b.nodes.size() && i < h.nodes.size() &&
+                        std::memcmp(&b.nodes[i], &h.nodes[i], sizeof(rm::Bvh8Node)) == 0;
+            for (int k = 0; same && k < 8; k++)
+                if (b.nodes[i].meta[k] && !((b.nodes[i].imask >> k) & 1))
+                    same = rm::leaf_ids(b, b.nodes[i], k) == rm::leaf_ids(h, h.nodes[i], k);
+            different += same ? 0u : 1u;
+        }
+        if (out_different) *out_different = different;
+        return 0;
+    } catch (const rm::HipError& e) {
+        if (err && err_cap) snprintf(err, err_cap, "%s", e.msg.c_str());
+        return -1;
+    } catch (const std::exception& e) {
+        if (err && err_cap) snprintf(err, err_cap, "%s", e.what());
+        return -1;
+    }
+}
 
 extern "C" int rmh_bvh8_check(const float* tris, uint32_t n, int threads, uint32_t* out_nodes, uint32_t* out_depth,
                               char* err, size_t err_cap) {
