@@ -1,7 +1,8 @@
 """The bounce loop's launches: closest hits merged with the previous bounce's
 shadow rays against separate launches (timing=1), streams that fit the queue
 (no regeneration, a known last iteration) and streams that do not, depths
-around the loop's chunks of iterations, against the oracle."""
+around the loop's chunks of iterations, against the oracle; two-level trees,
+lens rays, batches and caches against their separate launches; job times."""
 import numpy as np
 import pytest
 
@@ -67,3 +68,73 @@ def test_job_times_include_the_last_shadow_rays(device):
         gaps.append(st.ms_total - st.makespan_ms)
     print("from the job's time to the end %.3f ms, shadow rays of an iteration %.3f ms" % (min(gaps), launch))
     assert min(gaps) < 0.5 * launch
+
+
+@pytest.fixture(scope="module")
+def kinds(device, cornell):
+    field = scenes.instanced_field(W, H, grid=4, shapes=3, level=2)
+    lamps = scenes.lamp_box(W, H)
+    for d in (field, lamps):
+        d.envmap_resolution = 64
+    return {"two-level": scenes.build_device_scene(device, field, two_level=True),
+            "lens": scenes.build_device_scene(device, lamps), "cornell": cornell[0]}
+
+
+@pytest.mark.parametrize("kind", ["two-level", "lens"])
+@pytest.mark.parametrize("spl,samples", [(5, 5), (2, 5)], ids=["fits", "regenerates"])
+def test_two_level_and_lens_launches(kinds, kind, spl, samples):
+    """The merged launch, direct and from a captured graph, against the
+    separate ones: the same rays at every depth, the same image up to the
+    order of its sums."""
+    ref = None
+    for timing, graph in ((1, 0), (0, 0), (0, 1)):
+        r = api.Renderer(kinds[kind], W, H, max_depth=9, samples_per_launch=spl)
+        if kind == "lens":
+            r.set_lens(api.lens_desc(scenes.singlet_lens(50.0, 2.8), stop_index=3, relative_stop=0.7,
+                                     camera_scale=0.01, spectral=True))
+        r.set_uniforms(timing=timing, use_graph=graph, rr_depth=64, material_sort=1)
+        st = r.execute(samples)
+        got = (list(st.rays), list(st.shadow_rays), st.total_rays), r.image()
+        assert st.shadow_total > 0
+        ref = ref or got
+        assert got[0] == ref[0]
+        parity.assert_radiance_close(got[1], ref[1])
+
+
+@pytest.mark.parametrize("queue,graph", [(0, 0), (2048, 0), (0, 1), (2048, 1)])
+def test_batch_launches(device, kinds, queue, graph):
+    """Jobs of several depths in a queue that holds them and in one that does not."""
+    scene = kinds["cornell"]
+    b = api.Batch(device, [(scene, 40, 24, 3, 9, 1), (scene, 24, 32, 7, 1, 2), (scene, 33, 17, 2, 20, 3)])
+    st = b.render(queue_paths=queue, rr_depth=3, timing=1)
+    ref = [b.image(j) for j in range(3)]
+    got = b.render(queue_paths=queue, rr_depth=3, use_graph=graph)
+    assert (got.closest_rays, got.shadow_rays) == (st.closest_rays, st.shadow_rays)
+    for j in range(3):
+        parity.assert_radiance_close(b.image(j), ref[j])
+    t = b.job_times()
+    assert np.all(t > 0.0) and got.makespan_ms == t.max() <= got.ms_total
+
+
+@pytest.mark.parametrize("spl", [8, 2], ids=["fits", "regenerates"])
+def test_cache_launches(device, kinds, spl):
+    """A training cache sees the same vertices; with fixed parameters the
+    frames through it are the same."""
+    counts, images = [], []
+    for timing in (1, 0):
+        c = api.RadianceCache(device, log2_table_size=12, seed=3, train_shift=2, batch_size=256)
+        r = api.Renderer(kinds["cornell"], W, H, max_depth=9, samples_per_launch=spl)
+        r.set_uniforms(timing=timing, rr_depth=64, material_sort=1)
+        r.set_cache(c, mode=1)
+        r.execute(8)
+        s = c.stats()
+        counts.append((s.queries, s.train_records, s.samples, s.steps))
+        assert np.isfinite(s.last_loss) and min(counts[-1]) > 0
+        c = api.RadianceCache(device, log2_table_size=12, seed=3)
+        r = api.Renderer(kinds["cornell"], W, H, max_depth=9, samples_per_launch=spl)
+        r.set_uniforms(timing=timing, rr_depth=64, material_sort=1)
+        r.set_cache(c, mode=2)
+        r.execute(8)
+        images.append(r.image())
+    assert counts[0] == counts[1]
+    parity.assert_radiance_close(images[1], images[0])
