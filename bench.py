@@ -518,7 +518,9 @@ def main():
                               "shade": round(totals["ms_shade"] / args.steps, 3),
                               "trace_any_shadow": round(totals["ms_any"] / args.steps, 3),
                               "of": "%d further steps with closest hits and shadow rays in launches of their own, "
-                                    "%.3f ms each" % (args.steps, stages_wall * 1e3 / args.steps)},
+                                    "%.3f ms each" % (args.steps, stages_wall * 1e3 / args.steps),
+                              "closest": int(stg.closest_total), "shadow": int(stg.shadow_total),
+                              "launches": int(stg.iterations)},
         "roofline": {"kernel": "trace_closest", "bound": "hbm", "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": None if traffic is None else round(traffic),
