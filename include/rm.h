@@ -69,7 +69,11 @@ typedef struct rm_device_info {
     char arch[32];
 } rm_device_info;
 
-/* Replaces MTLCreateSystemDefaultDevice (Main.swift:22). */
+/* Replaces MTLCreateSystemDefaultDevice (Main.swift:22).  A device keeps until
+ * rm_device_destroy what its objects' calls share: after the first copy of 3 MB
+ * or more to or from ordinary host memory, 32 MB of pinned memory and up to
+ * eight threads that copy; after rm_trace_closest or rm_trace_any, their ray
+ * and hit buffers of up to 256 MB each. */
 int rm_device_create(int ordinal, rm_device** out);
 void rm_device_destroy(rm_device* dev);
 int rm_device_get_info(rm_device* dev, rm_device_info* out);

@@ -14,8 +14,10 @@
 //           (2^n - 1) << 5 | off    leaf with n in 1..3 triangles at
 //                                   tri_base + off (off + n <= 24)
 // Child slots are assigned so that slot k holds the child nearest to corner k
-// of the node (bit a of k set = high side on axis a); a ray with direction
-// octant `oct` visits internal children in order slot = k ^ oct, k = 0..7.
+// of the node (bit a of k set = high side on axis a).  The one-ray form
+// (bvh2l.h) visits internal children in order slot = k ^ oct, k = 0..7, for a
+// ray with direction octant `oct`; the kernels (kernels/trace.hip) take the
+// nearest child first, any hit the first in slot order.
 #pragma once
 #include "common.h"
 

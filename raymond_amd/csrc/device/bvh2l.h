@@ -13,15 +13,17 @@
 // closest over all instances, ties to the smaller (instance, primitive) as
 // in the flat tree.
 //
-// The traversal keeps one stack entry per tree level, as the flat kernels
-// do: a node group (child base, remaining child hits in visit order << 24 |
-// internal mask).  Entering an instance pushes the top-level group and a
-// marker entry holding the remaining instances of the leaf set; popping the
-// marker restores the world ray.  traverse2l below is the one-ray form that
-// the host check of the build runs (rmh_two_level_trace); the GPU kernels
-// take the same entry and exit steps inside their per-lane step machine
-// (RayState::enter and the marker pop in kernels/trace.hip), with the
-// postponed leaves and lane refill of the flat kernels.
+// A traversal keeps one stack entry per tree level, a node group (child base,
+// remaining child hits << 24 | internal mask).  Entering an instance pushes a
+// marker entry above the top-level group, holding the remaining instances of
+// the leaf set; popping the marker restores the world ray.  traverse2l below
+// is the one-ray form that the host check of the build runs
+// (rmh_two_level_trace), with a group's hits in the visit order of the ray's
+// octant.  The GPU kernels enter and leave instances in the same way
+// (RayState::enter and the marker pop in kernels/trace.hip), but visit the
+// nearest child first: their groups hold hits in slot order and the least
+// entry distance among them (bits 8 to 22), and they hold a lane's leaf sets
+// back for phases that many lanes take together.
 #pragma once
 #include "bvh.h"
 #include "isect.h"

@@ -5,6 +5,12 @@
 // the DMA's 0.6 ms.  HostCopies moves such copies in blocks through a ring of
 // pinned slots, where the DMA of one block overlaps the memcpy of others by a
 // few worker threads.
+//
+// The first copy of 3 MB or more sets this up: 32 MB of pinned slots, four
+// events, up to eight threads, kept until the device is destroyed.  Reading a
+// 1920x1080 image takes 10.2-10.8 ms the first time in a process and 1.3-1.45
+// later; plain copies, whose own staging the runtime sets up, took 15.8-16.2
+// and 2.5.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <condition_variable>

@@ -12,12 +12,13 @@
 //
 // The host builder takes 0.84 s for 1.3M triangles (16 threads, upload
 // included); this one takes 5.4 ms: 0.9 phase 1, 0.6 phase 2, 1.3 phase 3,
-// 1.5 phase 5, the rest set-up, allocation and the gaps between its 100 launches.  Phases 1 and 5
-// wait on memory and launches, phases 2 and 3 on their own split arithmetic.
+// 1.5 phase 5, the rest set-up, allocation and the gaps between its 100
+// launches.  Phases 1 and 5 wait on memory and launches, phases 2 and 3 on
+// their own split arithmetic.
 // Triangles are 32-byte records (bounds, id) that partitions move, so every
 // pass reads them in order:
 //   1. ranges above kBig records: level by level, several workgroups per
-//      range (bins and child bounds through global atomics);
+//      range (bins through global atomics, bounds as one partial union each);
 //   2. ranges of kSmall+1..kBig records: one workgroup builds a range down
 //      to kSmall records, bins in LDS, with its own stack of ranges;
 //   3. ranges of at most kSmall = 64 records: one wave builds the whole

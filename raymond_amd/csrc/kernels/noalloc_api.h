@@ -10,7 +10,7 @@ struct rm_scene;
 namespace rm {
 
 // Rays per rm_trace_closest_noalloc call; the library's fixed device array
-// holds 8 words per ray plus a 256-byte head (8.4 MB per GPU).
+// holds 8 words per ray plus the work counters (1 KB): 8.4 MB per GPU.
 constexpr uint32_t kNoAllocMaxRays = 1u << 18;
 
 // Takes the device address of the fixed array on the current device (called

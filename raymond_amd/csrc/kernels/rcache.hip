@@ -694,8 +694,9 @@ __global__ void rc_table_master_kernel(float* state, float* master, uint32_t* ta
 // Table gradients as the caller reads them: FP32, unscaled, from the scaled
 // FP16 sums, which are cleared for the next step.  Four pairs a thread; only
 // pairs that a sample touched are written back.  The host converted them
-// before: a gradients call on 8192 rows with the 2^19 table took 41.6 ms, and
-// takes 6.6 (64 MiB of gradients to the host; this pass moves 100 MB in HBM).
+// before: a gradients call on 8192 rows with the 2^19 table took 41.6 ms, with
+// this pass 6.6, and 1.75 since transfer.cpp brings the 64 MiB of gradients to
+// the host (the pass itself moves 100 MB in HBM).
 __global__ void rc_table_grads_kernel(uint32_t* grad_h2, float* out, size_t quads) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     const float unscale = 1.0f / kRcTableGradScale;

@@ -275,7 +275,7 @@ struct RayState {
                 tg = make_uint2(e.x, e.y & ~kMarker2l);
                 if (tg.y == 0u) set_ray(stk.world_o(), stk.world_d());
                 top = true;
-                        return false;
+                return false;
             }
             const uint32_t hits = e.y >> 24;
             const uint32_t rest = hits & (hits - 1u);
@@ -397,12 +397,10 @@ struct RayState {
 
     // Tests up to kTrisPerPhase postponed triangles; true when an any-hit
     // query found a hit.  Bounding the phase frees a lane with few triangles
-    // left for node steps while others still have some.  On the 5.2M-triangle
-    // sphere field (Mrays/s), one leaf slot: 1 per phase 2841, 2 per phase
-    // 2909, 3 2891, 4 2870, emptying every lane's list per phase slower than
-    // 1; two slots: 1 2899, 2 3033-3071, 3 3052.  Three per phase with the
-    // phase started at 1/4, 1/5 or 1/8 of the lanes held measured 3050-3084
-    // against 3104-3109 for two at 1/6 (the same box).
+    // left for node steps while others still have some.  With 1, 2, 3 and 4
+    // per phase the 5.2M-triangle sphere field (two leaf slots) measures
+    // 3675-3705, 3768-3774, 3793-3796 and 3776-3790 Mrays/s, the instanced
+    // field (one slot) 2744, 2845-2849, 2828-2830 and 2819-2823.
 #ifndef RM_TRIS_PER_PHASE
 #define RM_TRIS_PER_PHASE 2
 #endif
@@ -447,26 +445,26 @@ struct RayState {
 };
 
 // Waves per SIMD the trace kernels ask the register allocator for.  Left
-// free they take 95 and 92 VGPRs (5 waves); asking for 6 gives 80 VGPRs
-// with 48 and 36 bytes of spills per lane, which measured 2311 against
-// 3079-3097 Mrays/s on the 5.2M-triangle sphere field.
+// free they take 91 (closest hit) and 85 VGPRs (any hit): 5 waves.  Asking
+// for 6 gives 80 VGPRs with 28 and 12 bytes of spills per lane: the closest
+// hits of the 5.2M-triangle sphere field then take 0.85 ms per spp, not 0.60.
 #ifndef RM_TRACE_MIN_WAVES
 #define RM_TRACE_MIN_WAVES 1
 #endif
 constexpr int kTraceMinWaves = RM_TRACE_MIN_WAVES;
-// The two-level kernels take 98 and 95 VGPRs left free (4 and 5 waves per
-// SIMD); held to 5 waves both fit without spills.  With the world ray still
-// in registers they took 103 and 101 free, and 5 waves with spills measured
-// 2331 against 2295 Mrays/s for 4 waves on the 1080p instanced field.
+// The two-level kernels are held to 5 waves, which they fit without spills:
+// they take 92 and 85 VGPRs, held or left free.
 #ifndef RM_TWO_LEVEL_MIN_WAVES
 #define RM_TWO_LEVEL_MIN_WAVES 5
 #endif
 constexpr int kTwoLevelMinWaves = RM_TWO_LEVEL_MIN_WAVES;
-// Both traversals in one kernel are held to the separate kernels' 5 waves.
+// Both traversals in one kernel are held to the separate kernels' 5 waves (92
+// VGPRs, two-level 93, no spills).
 constexpr int kBothMinWaves = 5;
 
-// Lanes are refilled once at least this many of a wave's 64 are idle
-// (with two leaf slots, 4, 12 and 16 measured within 1% of 8).
+// Lanes are refilled once at least this many of a wave's 64 are idle (4, 8, 12
+// and 16 measure 3785, 3771, 3788 and 3777 Mrays/s on the sphere field, 2808,
+// 2847, 2842 and 2819 on the instanced field).
 #ifndef RM_REFILL_LANES
 #define RM_REFILL_LANES 8
 #endif
