@@ -8,6 +8,7 @@
 #include <thread>
 #include <tuple>
 #include <map>
+#include <memory>
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -672,6 +673,15 @@ void trace_closest_raw(rm_scene* s, const float* rays, uint32_t n, float* t, uin
     a.spill = s->d_spill.as<uint2>();
     const int blocks = s->dev->props.multiProcessorCount * s->dev->trace_blocks_per_cu;
     RM_HIP(launch_trace_closest(a, blocks, false, st));
+    if (5 * col <= kOneCopyMax) {
+        const std::unique_ptr<char[]> h(new char[5 * col]);
+        s->dev->copies->to_host({{h.get(), o, 5 * col}}, st);
+        if (bary) std::memcpy(bary, h.get(), 2 * col);
+        if (t) std::memcpy(t, h.get() + 2 * col, col);
+        if (inst) std::memcpy(inst, h.get() + 3 * col, col);
+        if (prim) std::memcpy(prim, h.get() + 4 * col, col);
+        return;
+    }
     std::vector<CopyPiece> hits;
     if (t) hits.push_back({t, a.hits.t, col});
     if (inst) hits.push_back({inst, a.hits.inst, col});

@@ -3,6 +3,8 @@ the 64 rays of a batch, one batch per persistent wave, and more.  A ray's hit
 does not depend on the batch it is in, so every batch is compared bit for bit
 with the same rays asked in blocks of 1000; the blocks' rays against the
 oracle."""
+import time
+
 import numpy as np
 import pytest
 
@@ -34,7 +36,7 @@ def traced(device, request):
     return scene, rays, closest, occluded
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 4097, 16383, 81921, 262143, 327679, 327681, 400000])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 4097, 16383, 52428, 52429, 81921, 262143, 327679, 327681, 400000])
 def test_batches_agree_at_every_size(traced, n):
     scene, rays, closest, occluded = traced
     got = scene.trace_closest(rays[:n])
@@ -66,3 +68,37 @@ def test_hit_arrays_may_overlap_the_rays(traced):
         hip.free()
     for g, c in zip(got, closest):
         assert np.array_equal(g.view(np.uint32), c[:n].view(np.uint32))
+
+
+def test_outputs_may_be_left_out(traced):
+    """Any of closest hits' arrays may be null, on both sides of the size from
+    which they are copied apart (52428 rays)."""
+    scene, rays, closest, _ = traced
+    for n in (100, 60000):
+        r = np.ascontiguousarray(rays[:n])
+        for keep in range(16):
+            got = [np.full(c[:n].shape, 7, c.dtype) for c in closest]
+            out = [g.ctypes.data if keep >> i & 1 else None for i, g in enumerate(got)]
+            assert api.LIB.rm_trace_closest(scene.handle, r.ctypes.data, n, *out) == 0
+            for i, (g, c) in enumerate(zip(got, closest)):
+                assert np.array_equal(g, c[:n]) if keep >> i & 1 else np.all(g == 7)
+
+
+def test_a_small_batch_costs_one_copy_back(traced):
+    """Closest hits have four arrays, any hits one: with one ray, a call of the
+    former that copies them apart takes twice as long as one of the latter
+    (64 against 31 us), in one copy as long (32)."""
+    scene = traced[0]
+    away = np.array([[0.0, 0.0, 100.0, 1e-3, 0.0, 0.0, 1.0, 1.0]], np.float32)  # no traversal
+
+    def least(call):
+        best = np.inf
+        for _ in range(300):
+            t = time.perf_counter()
+            call(away)
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    closest, any_hit = least(scene.trace_closest), least(scene.trace_any)
+    print("closest %.1f us, any %.1f us" % (closest * 1e6, any_hit * 1e6))
+    assert closest < 1.6 * any_hit
