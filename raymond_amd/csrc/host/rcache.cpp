@@ -1,6 +1,8 @@
 // Radiance cache, host side: parameter set-up, the Adam step sequence and the
 // raw-batch entry points.
 #include <cmath>
+#include <cstring>
+#include <memory>
 #include <vector>
 
 #include "rcache_host.h"
@@ -207,12 +209,22 @@ void cache_infer_raw(rm_cache* c, const float* features, uint32_t n, float* out)
 }
 
 static RcSamples stage_samples(rm_cache* c, const float* features, const float* targets, uint32_t n) {
-    stage_rows(c, c->stage_feat, features, (size_t)n * kRcFeatureFloats);
-    stage_rows(c, c->stage_target, targets, (size_t)n * 3);
+    const size_t nf = (size_t)n * kRcFeatureFloats, nt = (size_t)n * 3;
     RcSamples smp{};
+    smp.count = n;
+    if ((nf + nt) * 4 <= kOneCopyMax) {
+        const std::unique_ptr<float[]> h(new float[nf + nt]);
+        std::memcpy(h.get(), features, nf * 4);
+        std::memcpy(h.get() + nf, targets, nt * 4);
+        stage_rows(c, c->stage_feat, h.get(), nf + nt);
+        smp.feat = c->stage_feat.as<float>();
+        smp.target = smp.feat + nf;
+        return smp;
+    }
+    stage_rows(c, c->stage_feat, features, nf);
+    stage_rows(c, c->stage_target, targets, nt);
     smp.feat = c->stage_feat.as<float>();
     smp.target = c->stage_target.as<float>();
-    smp.count = n;
     return smp;
 }
 

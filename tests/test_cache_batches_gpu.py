@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 LOG2 = 12
 
 
-@pytest.mark.parametrize("n", [1, 31, 32, 33, 129])
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 129, 17476, 17477])
 def test_rows_at_tile_edges(device, n):
     rng = np.random.default_rng(n)
     mlp, table = random_params(rng, LOG2)
